@@ -24,6 +24,14 @@ template <typename R> struct Side {
     R t1, t2;
 };
 
+// x / 3, correctly rounded (the quotient corrected by its exact remainder).
+template <typename R> __device__ __forceinline__ R third(R x) { return x / R(3); }
+template <> __device__ __forceinline__ double third<double>(double x)
+{
+    const double q = x * (1.0 / 3.0);
+    return fma(fma(-3.0, q, x), 1.0 / 3.0, q);
+}
+
 // Solve one octant.  ordr/ordx/ordz in {0,1,2}, not all zero.
 template <typename R>
 __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, const Side<R>& sz,
@@ -50,7 +58,10 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
         for (int a = 0; a < 3; ++a)
             if (a != L && ord[a]) { if (o0 < 0) o0 = a; else o1 = a; }
     }
-    const R cL = ord[L] == 2 ? R(3) : R(1);
+    // cL is 3 only when every present axis is second order (a first-order one
+    // leads otherwise), so the ratio of an axis' coefficient to it is 1, or the
+    // axis' own: no division
+    const bool lead2 = ord[L] == 2;
     const R DL = ord[L] == 2 ? R(4) * t1[L] - t2[L] : t1[L];
     const R HL = ord[L] == 2 ? R(2) * h[L] : h[L];
     const R u2 = HL * HL, s2 = slown * slown;
@@ -61,7 +72,7 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
         const R ca0 = ord[o0] == 2 ? R(3) : R(1);
         const R Da0 = ord[o0] == 2 ? R(4) * t1[o0] - t2[o0] : t1[o0];
         const R Ha0 = ord[o0] == 2 ? R(2) * h[o0] : h[o0];
-        const R m0 = ca0 / cL;
+        const R m0 = lead2 ? R(1) : ca0;
         const R e0 = m0 * DL - Da0;
         const R H20 = Ha0 * Ha0;
         if (o1 < 0) {
@@ -72,7 +83,7 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
             const R ca1 = ord[o1] == 2 ? R(3) : R(1);
             const R Da1 = ord[o1] == 2 ? R(4) * t1[o1] - t2[o1] : t1[o1];
             const R Ha1 = ord[o1] == 2 ? R(2) * h[o1] : h[o1];
-            const R m1 = ca1 / cL;
+            const R m1 = lead2 ? R(1) : ca1;
             const R e1 = m1 * DL - Da1;
             const R H21 = Ha1 * Ha1;
             a = H20 * H21 + m0 * m0 * u2 * H21 + m1 * m1 * u2 * H20;
@@ -83,7 +94,36 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
     R disc = b * b - R(4) * a * c;
     if (disc < R(0)) disc = R(0);
     const R X = (-b + sqrt(disc)) / (R(2) * a);
-    return (DL + X) / cL;
+    return lead2 ? third<R>(DL + X) : DL + X;
+}
+
+// Whether one octant's solution T is certain to be the least of those of a
+// node no axis of which has both its sides counted (r, x, z: the counted
+// side of each axis, or an absent one).  The other octants' equations leave
+// out some of this one's squared terms ((c T - D) / H)^2, so at T their left
+// sides fall short of s^2 by the terms left out: with no term below a margin
+// well above the rounding of the whole sum, their larger roots lie beyond T
+// in the computed values too, and the minimum over the octants is T to the
+// last bit.  The sum's rounding is bounded by a few units in the last place
+// of 2 A T^2 + s^2 (times are absolute: T carries every other term); the
+// margin is 2^13 of them.  ih: the reciprocal spacings (any rounding).
+__device__ __forceinline__ bool octant_leads(const Side<double>& r, const Side<double>& x, const Side<double>& z,
+                                             double T, double ihr, double ihx, double ihz, double slown)
+{
+    const Side<double>* s[3] = { &r, &x, &z };
+    const double ih[3] = { ihr, ihx, ihz };
+    double A = 0.0, least = __builtin_huge_val();
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool two = s[a]->ord == 2;
+        const double num = two ? fma(1.5, T, fma(-2.0, s[a]->t1, 0.5 * s[a]->t2)) : T - s[a]->t1;
+        const double g = num * ih[a], al = two ? 1.5 * ih[a] : ih[a];
+        if (s[a]->ord > 0) {
+            A = fma(al, al, A);
+            least = fmin(least, g * g);
+        }
+    }
+    return least > 0x1p-40 * fma(2.0 * A * T, T, slown * slown);
 }
 
 // Minimum over the valid octants of a node whose six sides are prepared.

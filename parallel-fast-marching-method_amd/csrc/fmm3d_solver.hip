@@ -544,67 +544,146 @@ template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return _
 // A = B = 0 and so T = 0 * inf = NaN, and the running minimum is fmin,
 // which passes over a NaN.  Values arrive shifted by the smallest counted
 // neighbour.
-// One node update from the gathered stencil (sides r-, r+, x-, x+, z-, z+).
-// FAST selects the axis-sum octant form; otherwise the reference's
-// leading-axis form in the CPU oracle's operation order.
-template <typename R, bool FAST, bool SHIFT>
-__device__ __forceinline__ R col_update(int fom, R tc, const R v1[6], const R v2[6], const bool in1[6],
-                                        const bool in2[6], const R h[3], const R ih[3], R slown)
+//
+// One octant usually decides: with at most one side counted per axis, the
+// octant of the counted sides has the least solution, since the others leave
+// out some of its squared terms and so reach s^2 later.  In the computed
+// values that is certain where each counted term (alpha T - beta)^2 exceeds
+// the rounding of the whole sum, a few units in the last place of
+// M = A T^2 + sum beta^2 + s^2; the margin asked for is 2^8 of them (2^-16 M).
+// Nodes without it, and nodes with both sides of an axis counted, take the
+// minimum over all eight octants, so every value is the eight octants' value.
+// Measured: 6 % of the wavefronts' passes hold such a node in the first sweep
+// of 50 float32 plane waves at 201^3, which went from 5.55 to 3.53 G VALU
+// instructions (13.9 to 12.5 ms); eight float64 sources at 31x110x140 went
+// from 9.0 to 5.4 ms, a local source at 61^3 from 53 to 30 ms.
+// One node update.  gather(v1, v2) gives the stencil: the first and second
+// neighbours' values on the sides r-, r+, x-, x+, z-, z+ (inf outside the
+// grid); in1 says whether a side's first neighbour exists.  FAST selects the
+// axis-sum octant form; otherwise the reference's leading-axis form in the
+// CPU oracle's operation order.  h, ih: spacings and their reciprocals along
+// r, x, z.  Nodes that need all octants gather their stencil again, so that
+// the sides the one octant does not use hold no registers across it.
+template <typename R, bool FAST, bool SHIFT, typename G>
+__device__ __forceinline__ R col_update(int fom, R tc, G gather, const bool in1[6], const R h[3], const R ih[3],
+                                        R slown)
 {
     const R inf = Lim<R>::inf();
-    bool cnt[6], sec[6];
+    auto counts = [&](R v1, R t) { return SHIFT ? (v1 <= t && v1 < inf) : (v1 < t); };
+    Side<R> p[3];   // per axis its counted side; ord 0: none
+    bool sure = true;
     R tb = inf;
+    {
+        R v1[6], v2[6];
+        gather(v1, v2);
 #pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        cnt[q] = in1[q] && (SHIFT ? (v1[q] <= tc && v1[q] < inf) : (v1[q] < tc));
-        sec[q] = cnt[q] && fom && in2[q] && v2[q] < inf && v1[q] > v2[q];
-        if (SHIFT && cnt[q] && v1[q] < tb) tb = v1[q];
+        for (int a = 0; a < 3; ++a) {
+            const bool lo = counts(v1[2 * a], tc), hi = counts(v1[2 * a + 1], tc);
+            const R t1 = lo ? v1[2 * a] : v1[2 * a + 1], t2 = lo ? v2[2 * a] : v2[2 * a + 1];
+            p[a].ord = lo || hi ? (fom && t1 > t2 ? 2 : 1) : 0;
+            p[a].t1 = t1;
+            p[a].t2 = t2;
+            if (SHIFT && p[a].ord && t1 < tb) tb = t1;
+            sure = sure && !(lo && hi);
+            if (SHIFT && lo && v1[2 * a + 1] < tb) tb = v1[2 * a + 1];   // the other side may count too
+        }
     }
-    if (SHIFT && !(tb < inf)) return inf;
+    if (!(p[0].ord | p[1].ord | p[2].ord)) return inf;
     const R sh = SHIFT ? tb : R(0);
     R best;
-    if (FAST) {
-        // per side (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side
-        // carries a = NaN so every octant through it fails the A > 0 test
-        const R nan = __builtin_nan("");
-        R ta[6], tbb[6], tc2[6];
+    if constexpr (FAST) {
+        R pa[3], pb[3], paa[3], pbb[3];
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            // selects on plain values keep this branch-free
-            const R t1 = v1[q] - sh, t2 = v2[q] - sh;
-            const R num = sec[q] ? fma(R(-0.5), t2, t1 + t1) : t1;
-            const R al = ih[q / 2] * (cnt[q] ? (sec[q] ? R(1.5) : R(1)) : R(0));
-            const R be = cnt[q] ? num * ih[q / 2] : R(0);
-            ta[q] = in1[q] ? al * al : nan;
-            tbb[q] = al * be;
-            tc2[q] = be * be;
+        for (int a = 0; a < 3; ++a) {
+            const R t1 = p[a].t1 - sh, t2 = p[a].t2 - sh;
+            const R num = p[a].ord == 2 ? fma(R(-0.5), t2, t1 + t1) : t1;
+            pa[a] = ih[a] * (p[a].ord == 2 ? R(1.5) : p[a].ord ? R(1) : R(0));
+            pb[a] = p[a].ord ? num * ih[a] : R(0);
+            paa[a] = pa[a] * pa[a];
+            pbb[a] = pb[a] * pb[a];
         }
         const R s2 = slown * slown;
-        tc2[0] -= s2; tc2[1] -= s2;
-        best = inf;
+        const R A = paa[0] + (paa[1] + paa[2]), B = pa[0] * pb[0] + (pa[1] * pb[1] + pa[2] * pb[2]);
+        const R bb = pbb[1] + pbb[2], C = (pbb[0] - s2) + bb;
+        R disc = fused_mul_sub(B, B, A * C);
+        disc = disc > R(0) ? disc : R(0);
+        best = (B + fast_sqrt(disc)) * fast_rcp(A);
+        const R M = fma(A * best, best, pbb[0] + bb + s2);
+        R least = inf;
 #pragma unroll
-        for (int j = 2; j < 4; ++j)
-#pragma unroll
-            for (int k = 4; k < 6; ++k) {
-                const R Axz = ta[j] + ta[k], Bxz = tbb[j] + tbb[k], Cxz = tc2[j] + tc2[k];
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const R A = ta[i] + Axz, B = tbb[i] + Bxz, C = tc2[i] + Cxz;
-                    R disc = fused_mul_sub(B, B, A * C);
-                    disc = disc > R(0) ? disc : R(0);
-                    best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
-                }
-            }
-    } else {
-        Side<R> sd[3][2];
-#pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            Side<R>& S = sd[q / 2][q % 2];
-            S.ord = !in1[q] ? -1 : (sec[q] ? 2 : (cnt[q] ? 1 : 0));
-            S.t1 = cnt[q] ? v1[q] - sh : R(0);
-            S.t2 = sec[q] ? v2[q] - sh : R(0);
+        for (int a = 0; a < 3; ++a) {
+            const R g = fma(pa[a], best, -pb[a]);
+            least = fmin(least, p[a].ord ? g * g : inf);
         }
-        best = octant_min<R>(sd, h[0], h[1], h[2], slown);
+        sure = sure && least > R(0x1p-16) * M;
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            p[a].t1 = p[a].ord ? p[a].t1 - sh : R(0);
+            p[a].t2 = p[a].ord == 2 ? p[a].t2 - sh : R(0);
+        }
+        best = octant_solve<R>(p[0], p[1], p[2], h[0], h[1], h[2], slown);
+        sure = sure && octant_leads(p[0], p[1], p[2], best, ih[0], ih[1], ih[2], slown);
+    }
+    if (!sure) {
+        best = inf;
+        if constexpr (FAST) {
+            asm volatile("" ::: "memory");   // the stencil is read again, not kept
+            R v1[6], v2[6];
+            gather(v1, v2);
+            // per side (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side
+            // carries a = NaN so every octant through it fails the A > 0 test
+            const R nan = __builtin_nan("");
+            const R s2 = slown * slown;
+            R ta[6], tbb[6], tc2[6];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                // selects on plain values keep this branch-free
+                const bool cnt = counts(v1[q], tc), sec = fom && v1[q] > v2[q];
+                const R t1 = v1[q] - sh, t2 = v2[q] - sh;
+                const R num = sec ? fma(R(-0.5), t2, t1 + t1) : t1;
+                const R al = ih[q / 2] * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
+                const R be = cnt ? num * ih[q / 2] : R(0);
+                ta[q] = in1[q] ? al * al : nan;
+                tbb[q] = al * be;
+                tc2[q] = be * be;
+            }
+            tc2[0] -= s2; tc2[1] -= s2;
+#pragma unroll
+            for (int j = 2; j < 4; ++j)
+#pragma unroll
+                for (int k = 4; k < 6; ++k) {
+                    const R Axz = ta[j] + ta[k], Bxz = tbb[j] + tbb[k], Cxz = tc2[j] + tc2[k];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const R A = ta[i] + Axz, B = tbb[i] + Bxz, C = tc2[i] + Cxz;
+                        R disc = fused_mul_sub(B, B, A * C);
+                        disc = disc > R(0) ? disc : R(0);
+                        best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
+                    }
+                }
+        } else {
+            // one octant after another, each reading its own sides again
+#pragma unroll 1
+            for (int o = 0; o < 8; ++o) {
+                asm volatile("" ::: "memory");
+                R v1[6], v2[6];
+                gather(v1, v2);
+                bool in = true;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    const bool hi = (o >> a) & 1;
+                    const R t1 = hi ? v1[2 * a + 1] : v1[2 * a], t2 = hi ? v2[2 * a + 1] : v2[2 * a];
+                    in = in && (hi ? in1[2 * a + 1] : in1[2 * a]);
+                    p[a].ord = counts(t1, tc) ? (fom && t1 > t2 ? 2 : 1) : 0;
+                    p[a].t1 = p[a].ord ? t1 - sh : R(0);
+                    p[a].t2 = p[a].ord == 2 ? t2 - sh : R(0);
+                }
+                if (!in || !(p[0].ord | p[1].ord | p[2].ord)) continue;
+                const R T = octant_solve<R>(p[0], p[1], p[2], h[0], h[1], h[2], slown);
+                if (T < best) best = T;
+            }
+        }
     }
     if (SHIFT && best < inf) best = tb + best;
     return best;
@@ -914,25 +993,20 @@ k_column(ColArgs<R> a)
                     const int ix = x0 + lx, iz = z0 + lz;
                     const int own = (lx + 2) * LZ + lz + 2;
                     const R tc = cur[own];
-                    R v1[6], v2[6];
-                    bool in1[6], in2[6];
-                    in1[0] = ir >= 1; in2[0] = ir >= 2;
-                    in1[1] = ir + 1 < snr; in2[1] = ir + 2 < snr;
-                    in1[2] = ix >= 1; in2[2] = ix >= 2;
-                    in1[3] = ix + 1 < snx; in2[3] = ix + 2 < snx;
-                    in1[4] = iz >= 1; in2[4] = iz >= 2;
-                    in1[5] = iz + 1 < snz; in2[5] = iz + 2 < snz;
-                    // side 0 is the layer above (ir-1), side 1 the one below (ir+1)
-                    v1[0] = down ? b1[pl] : u1[pl]; v2[0] = down ? b2[pl] : u2[pl];
-                    v1[1] = down ? u1[pl] : b1[pl]; v2[1] = down ? u2[pl] : b2[pl];
-                    v1[2] = cur[own - LZ]; v2[2] = cur[own - 2 * LZ];
-                    v1[3] = cur[own + LZ]; v2[3] = cur[own + 2 * LZ];
-                    v1[4] = cur[own - 1]; v2[4] = cur[own - 2];
-                    v1[5] = cur[own + 1]; v2[5] = cur[own + 2];
-                    rst.apply(v1, v2);
+                    const bool in1[6] = { ir >= 1, ir + 1 < snr, ix >= 1, ix + 1 < snx, iz >= 1, iz + 1 < snz };
+                    auto gather = [&](R v1[6], R v2[6]) {
+                        // side 0 is the layer above (ir-1), side 1 the one below (ir+1)
+                        v1[0] = down ? b1[pl] : u1[pl]; v2[0] = down ? b2[pl] : u2[pl];
+                        v1[1] = down ? u1[pl] : b1[pl]; v2[1] = down ? u2[pl] : b2[pl];
+                        v1[2] = cur[own - LZ]; v2[2] = cur[own - 2 * LZ];
+                        v1[3] = cur[own + LZ]; v2[3] = cur[own + 2 * LZ];
+                        v1[4] = cur[own - 1]; v2[4] = cur[own - 2];
+                        v1[5] = cur[own + 1]; v2[5] = cur[own + 2];
+                        rst.apply(v1, v2);
+                    };
                     const R h[3] = { hr, hxl, shz[lx] };
                     const R ih[3] = { ihr, ihx, sihz[lx] };
-                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, v1, v2, in1, in2, h, ih, slown), rq);
+                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, in1, h, ih, slown), rq);
                     // every lane has read its stencil before any lane writes (one wavefront)
                     __builtin_amdgcn_wave_barrier();
                     if (nv != tc) {
@@ -1088,24 +1162,21 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         for (int ir = 0; ir < snr; ++ir) {
             const size_t c = (size_t)ir * NL + f;
             if (!((fb[c >> 5] >> (c & 31)) & 1u)) {
-                R v1[6], v2[6];
-                bool in1[6], in2[6];
-                in1[0] = ir >= 1; in2[0] = ir >= 2;
-                in1[1] = ir + 1 < snr; in2[1] = ir + 2 < snr;
-                in1[2] = ix >= 1; in2[2] = ix >= 2;
-                in1[3] = ix + 1 < snx; in2[3] = ix + 2 < snx;
-                in1[4] = iz >= 1; in2[4] = iz >= 2;
-                in1[5] = iz + 1 < snz; in2[5] = iz + 2 < snz;
+                const bool in1[6] = { ir >= 1, ir + 1 < snr, ix >= 1, ix + 1 < snx, iz >= 1, iz + 1 < snz };
+                rst.layer(rs, ir, snr);
                 // side 0 the layer above (ir-1), side 1 the one below (ir+1);
                 // out of the grid reads as inf, as the walk's staging does
-                v1[0] = w[1]; v2[0] = w[0];
-                v1[1] = w[3]; v2[1] = w[4];
-                v1[2] = in1[2] ? T[c - a.nnz] : inf; v2[2] = in2[2] ? T[c - 2 * (size_t)a.nnz] : inf;
-                v1[3] = in1[3] ? T[c + a.nnz] : inf; v2[3] = in2[3] ? T[c + 2 * (size_t)a.nnz] : inf;
-                v1[4] = in1[4] ? T[c - 1] : inf; v2[4] = in2[4] ? T[c - 2] : inf;
-                v1[5] = in1[5] ? T[c + 1] : inf; v2[5] = in2[5] ? T[c + 2] : inf;
-                rst.layer(rs, ir, snr);
-                rst.apply(v1, v2);
+                auto gather = [&](R v1[6], R v2[6]) {
+                    v1[0] = w[1]; v2[0] = w[0];
+                    v1[1] = w[3]; v2[1] = w[4];
+                    v1[2] = ix >= 1 ? T[c - a.nnz] : inf; v2[2] = ix >= 2 ? T[c - 2 * (size_t)a.nnz] : inf;
+                    v1[3] = ix + 1 < snx ? T[c + a.nnz] : inf; v2[3] = ix + 2 < snx ? T[c + 2 * (size_t)a.nnz] : inf;
+                    v1[4] = iz >= 1 ? T[c - 1] : inf; v2[4] = iz >= 2 ? T[c - 2] : inf;
+                    v1[5] = iz + 1 < snz ? T[c + 1] : inf; v2[5] = iz + 2 < snz ? T[c + 2] : inf;
+                    rst.apply(v1, v2);
+                };
+                R v1[6], v2[6];
+                gather(v1, v2);
                 // the lowest input relaxed after the node, in its frame
                 R lm = down ? fmin(v1[1], v2[1]) : fmin(v1[0], v2[0]);
                 if (late_x[0]) lm = fmin(lm, v1[2]);
@@ -1120,7 +1191,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
                     const R hxl = a.hx[slot * a.geo_hx + ir], hzl = a.hz[slot * a.geo_hz + (size_t)ir * a.nnx + ix];
                     const R h[3] = { hr, hxl, hzl };
                     const R ih[3] = { ihr, R(1) / hxl, R(1) / hzl };
-                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, w[2], v1, v2, in1, in2, h, ih, a.slo[slot * a.geo_n + c]), qs);
+                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, w[2], gather, in1, h, ih, a.slo[slot * a.geo_n + c]), qs);
                     if (nv != w[2] && !(fabs(nv - w[2]) <= vtl)) moved = true;
                 }
             }
@@ -1390,20 +1461,19 @@ k_plane(ColArgs<R> a)
                 const bool fixed = (qf[q] >> (c & 31)) & 1u;
                 if (!fixed) {
                     const int ir = down ? w : nr - 1 - w;
-                    R v1[6], v2[6];
-                    bool in1[6], in2[6];
                     // side 0 is layer ir-1, side 1 layer ir+1; the walk reached ir from ir+1 (up) or ir-1 (down)
-                    v1[0] = down ? P1 : N1; v2[0] = down ? P2 : N2;
-                    v1[1] = down ? N1 : P1; v2[1] = down ? N2 : P2;
-                    v1[2] = xm1; v2[2] = xm2; v1[3] = xp1; v2[3] = xp2;
-                    v1[4] = zm1; v2[4] = zm2; v1[5] = zp1; v2[5] = zp2;
-                    in1[0] = ir >= 1; in2[0] = ir >= 2;
-                    in1[1] = ir + 1 < nr; in2[1] = ir + 2 < nr;
-                    in1[2] = lf & 1u; in2[2] = lf & 2u; in1[3] = lf & 4u; in2[3] = lf & 8u;
-                    in1[4] = lf & 16u; in2[4] = lf & 32u; in1[5] = lf & 64u; in2[5] = lf & 128u;
+                    auto gather = [&](R v1[6], R v2[6]) {
+                        v1[0] = down ? P1 : N1; v2[0] = down ? P2 : N2;
+                        v1[1] = down ? N1 : P1; v2[1] = down ? N2 : P2;
+                        v1[2] = xm1; v2[2] = xm2; v1[3] = xp1; v2[3] = xp2;
+                        v1[4] = zm1; v2[4] = zm2; v1[5] = zp1; v2[5] = zp2;
+                    };
+                    bool in1[6] = { ir >= 1, ir + 1 < nr, false, false, false, false };
+                    in1[2] = lf & 1u; in1[3] = lf & 4u;
+                    in1[4] = lf & 16u; in1[5] = lf & 64u;
                     const R h[3] = { hr, qhx[q], qhz[q] };
                     const R ih[3] = { ihr, fast_rcp(qhx[q]), fast_rcp(qhz[q]) };
-                    const R nv = col_update<R, FAST, SHIFT>(a.fom, C0, v1, v2, in1, in2, h, ih, qs[q]);
+                    const R nv = col_update<R, FAST, SHIFT>(a.fom, C0, gather, in1, h, ih, qs[q]);
                     ++nupd;
                     if (nv != C0) {
                         cur = nv;
