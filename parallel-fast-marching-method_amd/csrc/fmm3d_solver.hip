@@ -3827,6 +3827,8 @@ static int solve_tele_part(fmm3d_ctx* c, const char* fn, int nsrc, const double*
         c->d_faces_n = (size_t)nsrc * F;
     }
     c->stg_n = 0;   // the staged faces are replaced
+    // no point sources: the rays run to the grid's faces
+    k_fill_real<double><<<(3 * nsrc + 255) / 256, 256, 0, c->stream>>>(c->sl.srcpos, (size_t)3 * nsrc, __builtin_nan(""));
     HIPCHK(c, hipMemcpyAsync(c->d_faces, faces, (size_t)nsrc * F * sizeof(double), hipMemcpyHostToDevice, c->stream));
     c->stats = fmm3d_stats{};
     HIPCHK(c, hipMemsetAsync(c->d_visits, 0, 3 * sizeof(unsigned long long), c->stream));
