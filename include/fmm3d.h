@@ -271,7 +271,9 @@ int fmm3d_get_stats(const fmm3d_ctx *ctx, fmm3d_stats *out);
  *   "point_warm"    refined blocks: 1 (default) a float32 solve first, then
  *                   float64 sweeps from its field to the float64 fixed
  *                   point; 0 float64 from the start
- *   "spin_limit"    polls before such a wait is given up (default 20000)
+ *   "spin_limit"    polls before such a wait is given up (default 20000;
+ *                   four times as many where the neighbour's progress is
+ *                   in the same XCD's cache)
  *   "check_every"   column walk: sweeps between convergence checks (1..8,
  *                   default 4); at a check, every source whose last sweep
  *                   changed nothing leaves the remaining sweeps

@@ -97,33 +97,63 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
     return lead2 ? third<R>(DL + X) : DL + X;
 }
 
-// Whether one octant's solution T is certain to be the least of those of a
-// node no axis of which has both its sides counted (r, x, z: the counted
-// side of each axis, or an absent one).  The other octants' equations leave
-// out some of this one's squared terms ((c T - D) / H)^2, so at T their left
-// sides fall short of s^2 by the terms left out: with no term below a margin
-// well above the rounding of the whole sum, their larger roots lie beyond T
-// in the computed values too, and the minimum over the octants is T to the
-// last bit.  The sum's rounding is bounded by a few units in the last place
-// of 2 A T^2 + s^2 (times are absolute: T carries every other term); the
-// margin is 2^13 of them.  ih: the reciprocal spacings (any rounding).
-__device__ __forceinline__ bool octant_leads(const Side<double>& r, const Side<double>& x, const Side<double>& z,
-                                             double T, double ihr, double ihx, double ihz, double slown)
+// The octant of one side per axis (ord 0: the axis is absent, t1 = t2 = 0),
+// as octant_solve gives it to the last bit, without its branches: an absent
+// axis enters the three-axis expressions as H^2 = 1 and m = e = 0, which
+// leaves the ones of two or one axis.  h2: squared spacings.  *weak: the axes
+// (bits) whose term is not certain; without any, this solution T is the least
+// over a node's octants when none of its axes has both sides counted.  The
+// other octants' equations leave out some of this one's squared terms ((c T - D) / H)^2, so at T their left
+// sides fall short of s^2 by the terms left out: where every term is above
+// the rounding of the whole sum, their larger roots lie beyond T in the
+// computed values too, and the minimum over the octants is T to the last bit.
+// A term must be positive (c T > D): the terms weighted by c / H sum to half
+// the equation's slope at T, which is then a root and not where the
+// discriminant was clamped.  The sum's rounding is a few units in the last
+// place of sum (c T / H)^2 + s^2 (times are absolute: T carries the other
+// terms); kt >= 2^-40 sum (c / H)^2 and ks = 2^-40 s^2 put the bound at 2^13
+// of them.
+__device__ __forceinline__ double octant_one(const Side<double> p[3], const double h2[3], double s2, double kt,
+                                             double ks, unsigned* weak)
 {
-    const Side<double>* s[3] = { &r, &x, &z };
-    const double ih[3] = { ihr, ihx, ihz };
-    double A = 0.0, least = __builtin_huge_val();
+    bool one[3], has[3];
+    double D[3], H2[3], c[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const bool two = s[a]->ord == 2;
-        const double num = two ? fma(1.5, T, fma(-2.0, s[a]->t1, 0.5 * s[a]->t2)) : T - s[a]->t1;
-        const double g = num * ih[a], al = two ? 1.5 * ih[a] : ih[a];
-        if (s[a]->ord > 0) {
-            A = fma(al, al, A);
-            least = fmin(least, g * g);
-        }
+        one[a] = p[a].ord == 1;
+        has[a] = p[a].ord != 0;
+        const bool two = p[a].ord == 2;
+        D[a] = two ? fma(4.0, p[a].t1, -p[a].t2) : p[a].t1;   // 4 t1 is exact
+        H2[a] = has[a] ? (two ? 4.0 * h2[a] : h2[a]) : 1.0;   // (2 h)^2 = 4 h^2 exactly
+        c[a] = two ? 3.0 : 1.0;
     }
-    return least > 0x1p-40 * fma(2.0 * A * T, T, slown * slown);
+    // the leading axis: the first first-order one, else the first present
+    const bool first = one[0] || one[1] || one[2];
+    const bool l0 = first ? one[0] : has[0], l1 = !l0 && (first ? one[1] : has[1]), l2 = !l0 && !l1;
+    const double DL = l0 ? D[0] : l1 ? D[1] : D[2], u2 = l0 ? H2[0] : l1 ? H2[1] : H2[2];
+    const double D0 = l1 ? D[0] : D[1], D1 = l2 ? D[0] : D[2];
+    const double H20 = l1 ? H2[0] : H2[1], H21 = l2 ? H2[0] : H2[2];
+    const double c0 = l1 ? c[0] : c[1], c1 = l2 ? c[0] : c[2];
+    const bool has0 = l1 ? has[0] : has[1], has1 = l2 ? has[0] : has[2];
+    const double m0 = has0 ? (first ? c0 : 1.0) : 0.0, m1 = has1 ? (first ? c1 : 1.0) : 0.0;
+    const double e0 = m0 * DL - D0, e1 = m1 * DL - D1;
+    const double qa = H20 * H21 + m0 * m0 * u2 * H21 + m1 * m1 * u2 * H20;
+    const double qb = 2.0 * u2 * (m0 * e0 * H21 + m1 * e1 * H20);
+    const double qc = u2 * (e0 * e0 * H21 + e1 * e1 * H20 - s2 * H20 * H21);
+    double disc = qb * qb - 4.0 * qa * qc;
+    if (disc < 0.0) disc = 0.0;
+    const double X = DL + (-qb + sqrt(disc)) / (2.0 * qa);
+    const double T = first ? X : third<double>(X);
+    const double thr = fma(kt * T, T, ks);
+    unsigned w = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        // an absent axis compares T^2 itself
+        const double g = fma(c[a], T, -D[a]);
+        w |= g * fabs(g) > thr * H2[a] ? 0u : 1u << a;
+    }
+    *weak = w;
+    return T;
 }
 
 // Minimum over the valid octants of a node whose six sides are prepared.

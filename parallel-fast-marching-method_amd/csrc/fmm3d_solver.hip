@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <limits>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -405,6 +406,7 @@ template <typename R> struct ColArgs {
     int nnr, nnx, nnz;
     int npx, npz;           // patches per axis
     int nslots;
+    const int* act;         // 8 x 8 patches: the slots of this sweep (k_next_sweep)
     int iter;
     int fom;
     int maxpass;            // line passes per layer at most (cycle +phi, -phi, +theta, -theta)
@@ -470,6 +472,36 @@ template <typename P> __device__ __forceinline__ P uniform_load(const P* p, size
     return ((const __attribute__((address_space(4))) P*)p)[i];
 }
 
+// The two sides of one axis of a node's stencil: the first and second
+// neighbours' values towards the lower index (l1, l2) and the higher one
+// (h1, h2), inf outside the grid, and whether the first ones exist.
+template <typename R> struct AxisSides {
+    R l1, l2, h1, h2;
+    bool lin, hin;
+};
+
+// Element i of p, p the same in every lane: with the lane's part a 32-bit
+// byte offset the address needs no 64-bit arithmetic per lane (an element
+// index times its size stays under 2^32: a layer's nodes).  The coherent
+// forms reach past the XCD's own L2.
+template <typename P> __device__ __forceinline__ P lane_load(const P* p, unsigned i)
+{
+    return *(const P*)((const char*)p + i * (unsigned)sizeof(P));
+}
+template <typename P> __device__ __forceinline__ P lane_load_coherent(const P* p, unsigned i)
+{
+    return __hip_atomic_load((const P*)((const char*)p + i * (unsigned)sizeof(P)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A store other patches read in the same sweep: to this XCD's L2 where every
+// patch that reads it runs on this XCD (local), past it otherwise.  (The end
+// of the kernel makes either visible to the whole device.)
+template <typename P> __device__ __forceinline__ void walk_store(P* p, unsigned i, P v, bool local)
+{
+    P* q = (P*)((char*)p + i * (unsigned)sizeof(P));
+    if (local) __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Steps of a slot's reference from node (ir, ix, iz) to its stencil
 // neighbours: a float32 neighbour value plus its step is the neighbour's
 // time relative to the centre node's reference.  Every step is a multiple
@@ -507,14 +539,17 @@ template <typename R> struct RefSteps {
         fetch(rs, ir, snr);
         settle(rs, ir, snr);
     }
-    // v1/v2 in side order r-, r+, x-, x+, z-, z+
-    __device__ __forceinline__ void apply(R v1[6], R v2[6]) const
+    // the sides of axis ax in the node's frame
+    __device__ __forceinline__ AxisSides<R> apply(AxisSides<R> g, int ax) const
     {
-        if (std::is_same<R, float>::value) {
-            v1[0] += up1; v2[0] += up2; v1[1] += dn1; v2[1] += dn2;
-            v1[2] -= gx; v2[2] -= gx + gx; v1[3] += gx; v2[3] += gx + gx;
-            v1[4] -= gz; v2[4] -= gz + gz; v1[5] += gz; v2[5] += gz + gz;
+        if constexpr (std::is_same<R, float>::value) {
+            if (ax == 0) { g.l1 += up1; g.l2 += up2; g.h1 += dn1; g.h2 += dn2; }
+            else {
+                const R s = ax == 1 ? gx : gz;
+                g.l1 -= s; g.l2 -= s + s; g.h1 += s; g.h2 += s + s;
+            }
         }
+        return g;
     }
 };
 
@@ -545,148 +580,183 @@ template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return _
 // which passes over a NaN.  Values arrive shifted by the smallest counted
 // neighbour.
 //
-// One octant usually decides: with at most one side counted per axis, the
+// One octant usually decides.  With at most one side counted per axis, the
 // octant of the counted sides has the least solution, since the others leave
 // out some of its squared terms and so reach s^2 later.  In the computed
-// values that is certain where each counted term (alpha T - beta)^2 exceeds
-// the rounding of the whole sum, a few units in the last place of
-// M = A T^2 + sum beta^2 + s^2; the margin asked for is 2^8 of them (2^-16 M).
-// Nodes without it, and nodes with both sides of an axis counted, take the
-// minimum over all eight octants, so every value is the eight octants' value.
-// Measured: 6 % of the wavefronts' passes hold such a node in the first sweep
-// of 50 float32 plane waves at 201^3, which went from 5.55 to 3.53 G VALU
-// instructions (13.9 to 12.5 ms); eight float64 sources at 31x110x140 went
-// from 9.0 to 5.4 ms, a local source at 61^3 from 53 to 30 ms.
-// One node update.  gather(v1, v2) gives the stencil: the first and second
-// neighbours' values on the sides r-, r+, x-, x+, z-, z+ (inf outside the
-// grid); in1 says whether a side's first neighbour exists.  FAST selects the
-// axis-sum octant form; otherwise the reference's leading-axis form in the
-// CPU oracle's operation order.  h, ih: spacings and their reciprocals along
-// r, x, z.  Nodes that need all octants gather their stencil again, so that
-// the sides the one octant does not use hold no registers across it.
-template <typename R, bool FAST, bool SHIFT, typename G>
-__device__ __forceinline__ R col_update(int fom, R tc, G gather, const bool in1[6], const R h[3], const R ih[3],
-                                        R slown)
+// values that is certain where each counted term alpha T - beta is positive
+// (so T is a root and not where the discriminant was clamped) and its square
+// exceeds the rounding of the whole sum, a few units in the last place of
+// M = A T^2 + sum beta^2 + s^2 <= 3 (sum beta^2 + s^2); the margin asked for
+// is 2^8 of them.  Where an axis' term is not certain, the octant without it
+// is evaluated too, and where both sides of an axis count, the octants of
+// either, so that every value is the minimum over all eight octants to the
+// last bit.  Measured against eight octants each time: 6 % of the wavefronts'
+// passes need more than one in the first sweep of 50 float32 plane waves at
+// 201^3, which went from 5.55 to 3.53 G VALU instructions; eight float64
+// sources at 31x110x140 went from 9.0 to 5.4 ms, a local source at 61^3 from
+// 53 to 30 ms.
+
+// The octant of one side per axis (ord 0: none; t1, t2 relative to a common
+// time), its solution and the axes whose term is not certain (bits).
+// h2: squared spacings; kt: as octant_one's (float64).
+template <typename R, bool FAST>
+__device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], const R ih[3], R s2, R kt, unsigned* weak)
 {
-    const R inf = Lim<R>::inf();
-    auto counts = [&](R v1, R t) { return SHIFT ? (v1 <= t && v1 < inf) : (v1 < t); };
-    Side<R> p[3];   // per axis its counted side; ord 0: none
-    bool sure = true;
-    R tb = inf;
-    {
-        R v1[6], v2[6];
-        gather(v1, v2);
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const bool lo = counts(v1[2 * a], tc), hi = counts(v1[2 * a + 1], tc);
-            const R t1 = lo ? v1[2 * a] : v1[2 * a + 1], t2 = lo ? v2[2 * a] : v2[2 * a + 1];
-            p[a].ord = lo || hi ? (fom && t1 > t2 ? 2 : 1) : 0;
-            p[a].t1 = t1;
-            p[a].t2 = t2;
-            if (SHIFT && p[a].ord && t1 < tb) tb = t1;
-            sure = sure && !(lo && hi);
-            if (SHIFT && lo && v1[2 * a + 1] < tb) tb = v1[2 * a + 1];   // the other side may count too
-        }
-    }
-    if (!(p[0].ord | p[1].ord | p[2].ord)) return inf;
-    const R sh = SHIFT ? tb : R(0);
-    R best;
     if constexpr (FAST) {
         R pa[3], pb[3], paa[3], pbb[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const R t1 = p[a].t1 - sh, t2 = p[a].t2 - sh;
-            const R num = p[a].ord == 2 ? fma(R(-0.5), t2, t1 + t1) : t1;
-            pa[a] = ih[a] * (p[a].ord == 2 ? R(1.5) : p[a].ord ? R(1) : R(0));
-            pb[a] = p[a].ord ? num * ih[a] : R(0);
+            const bool cnt = p[a].ord != 0, sec = p[a].ord == 2;
+            const R num = sec ? fma(R(-0.5), p[a].t2, p[a].t1 + p[a].t1) : p[a].t1;
+            pa[a] = ih[a] * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
+            pb[a] = cnt ? num * ih[a] : R(0);
             paa[a] = pa[a] * pa[a];
             pbb[a] = pb[a] * pb[a];
         }
-        const R s2 = slown * slown;
         const R A = paa[0] + (paa[1] + paa[2]), B = pa[0] * pb[0] + (pa[1] * pb[1] + pa[2] * pb[2]);
         const R bb = pbb[1] + pbb[2], C = (pbb[0] - s2) + bb;
         R disc = fused_mul_sub(B, B, A * C);
         disc = disc > R(0) ? disc : R(0);
-        best = (B + fast_sqrt(disc)) * fast_rcp(A);
-        const R M = fma(A * best, best, pbb[0] + bb + s2);
-        R least = inf;
+        const R T = (B + fast_sqrt(disc)) * fast_rcp(A);
+        const R thr = R(0x1.8p-15) * (pbb[0] + bb + s2);
+        unsigned w = 0;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const R g = fma(pa[a], best, -pb[a]);
-            least = fmin(least, p[a].ord ? g * g : inf);
+            const R g = fma(pa[a], T, -pb[a]);
+            w |= (p[a].ord != 0 && !(g * fabs(g) > thr)) ? 1u << a : 0u;
         }
-        sure = sure && least > R(0x1p-16) * M;
+        *weak = w;
+        return T;
     } else {
+        return octant_one(p, h2, s2, kt, R(0x1p-40) * s2, weak);
+    }
+}
+
+// The minimum over the octants of a node whose one octant was not certain
+// (sides counted below top, times relative to sh).  Per axis, role 0 is the
+// lower side and role 1 the other: its octants differ where both sides count
+// (both), and where role 1 leaves the axis out while role 0 counts (drop).
+// In float64 the octants of the counted sides come first, then those without
+// one or more of the axes some of them left uncertain (eight float64 plane
+// waves at 31x110x140, first sweep: 5.2 ms with all eight octants there, 3.3
+// with these; float32 at 201^3 was slower, 8.6 against 12.0 ms).  The stencil is gathered again for
+// each, so that this path holds few registers.
+template <typename R, bool FAST, bool SHIFT, typename G>
+__device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const R h2[3], const R ih[3], R s2, R kt)
+{
+    auto counts = [&](R v) { return SHIFT ? v <= top : v < top; };
+    R best = Lim<R>::inf();
+    if constexpr (FAST) {
+        // an octant is cheap here (a hardware square root and reciprocal):
+        // all eight, one theta side and one phi side at a time.  Per side
+        // (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side carries
+        // a = NaN, and fmin passes over the octants through it
+        struct Coef { R a, b, c; };
+        auto coef = [&](R w1, R w2, bool in, R ihx) {
+            // selects on plain values keep this branch-free
+            const bool cnt = counts(w1), sec = fom && w1 > w2;
+            const R u1 = w1 - sh, u2 = w2 - sh;
+            const R num = sec ? fma(R(-0.5), u2, u1 + u1) : u1;
+            const R al = ihx * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
+            const R be = cnt ? num * ihx : R(0);
+            return Coef{ in ? al * al : R(__builtin_nan("")), al * be, be * be };
+        };
+#pragma unroll 1
+        for (int o = 0; o < 4; ++o) {
+            asm volatile("" ::: "memory");   // the stencil is read again, not kept
+            const AxisSides<R> r = gather(0), x = gather(1), z = gather(2);
+            const bool hx = o & 1, hz = o & 2;
+            const Coef cx = coef(hx ? x.h1 : x.l1, hx ? x.h2 : x.l2, hx ? x.hin : x.lin, ih[1]);
+            const Coef cz = coef(hz ? z.h1 : z.l1, hz ? z.h2 : z.l2, hz ? z.hin : z.lin, ih[2]);
+            const Coef c0 = coef(r.l1, r.l2, r.lin, ih[0]), c1 = coef(r.h1, r.h2, r.hin, ih[0]);
+            const R Axz = cx.a + cz.a, Bxz = cx.b + cz.b, Cxz = cx.c + cz.c;
+            auto octant = [&](const Coef& c) {
+                const R A = c.a + Axz, B = c.b + Bxz, C = (c.c - s2) + Cxz;
+                R disc = fused_mul_sub(B, B, A * C);
+                disc = disc > R(0) ? disc : R(0);
+                best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
+            };
+            octant(c0);
+            octant(c1);
+        }
+        return best;
+    }
+    unsigned both = 0, drop = 0, unsure = 0;
+#pragma unroll 1
+    for (int j = 0; j < 16; ++j) {
+        const unsigned m = j & 7;   // role 1 on these axes
+        const bool first = j < 8;   // counted sides only
+        if (j > 0 && !(first ? (m & ~both) == 0 : (m & ~(both | unsure)) == 0 && (m & unsure))) continue;
+        asm volatile("" ::: "memory");
+        Side<R> p[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            p[a].t1 = p[a].ord ? p[a].t1 - sh : R(0);
-            p[a].t2 = p[a].ord == 2 ? p[a].t2 - sh : R(0);
-        }
-        best = octant_solve<R>(p[0], p[1], p[2], h[0], h[1], h[2], slown);
-        sure = sure && octant_leads(p[0], p[1], p[2], best, ih[0], ih[1], ih[2], slown);
-    }
-    if (!sure) {
-        best = inf;
-        if constexpr (FAST) {
-            asm volatile("" ::: "memory");   // the stencil is read again, not kept
-            R v1[6], v2[6];
-            gather(v1, v2);
-            // per side (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side
-            // carries a = NaN so every octant through it fails the A > 0 test
-            const R nan = __builtin_nan("");
-            const R s2 = slown * slown;
-            R ta[6], tbb[6], tc2[6];
-#pragma unroll
-            for (int q = 0; q < 6; ++q) {
-                // selects on plain values keep this branch-free
-                const bool cnt = counts(v1[q], tc), sec = fom && v1[q] > v2[q];
-                const R t1 = v1[q] - sh, t2 = v2[q] - sh;
-                const R num = sec ? fma(R(-0.5), t2, t1 + t1) : t1;
-                const R al = ih[q / 2] * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
-                const R be = cnt ? num * ih[q / 2] : R(0);
-                ta[q] = in1[q] ? al * al : nan;
-                tbb[q] = al * be;
-                tc2[q] = be * be;
+            const AxisSides<R> g = gather(a);
+            const bool lo = g.l1 <= g.h1, one = (m >> a) & 1;
+            const R o1 = lo ? g.h1 : g.l1, o2 = lo ? g.h2 : g.l2, q1 = lo ? g.l1 : g.h1, q2 = lo ? g.l2 : g.h2;
+            const bool ob = counts(o1);
+            if (j == 0) {
+                both |= ob ? 1u << a : 0u;
+                drop |= !ob && counts(q1) && (lo ? g.hin : g.lin) ? 1u << a : 0u;
             }
-            tc2[0] -= s2; tc2[1] -= s2;
-#pragma unroll
-            for (int j = 2; j < 4; ++j)
-#pragma unroll
-                for (int k = 4; k < 6; ++k) {
-                    const R Axz = ta[j] + ta[k], Bxz = tbb[j] + tbb[k], Cxz = tc2[j] + tc2[k];
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const R A = ta[i] + Axz, B = tbb[i] + Bxz, C = tc2[i] + Cxz;
-                        R disc = fused_mul_sub(B, B, A * C);
-                        disc = disc > R(0) ? disc : R(0);
-                        best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
-                    }
-                }
-        } else {
-            // one octant after another, each reading its own sides again
-#pragma unroll 1
-            for (int o = 0; o < 8; ++o) {
-                asm volatile("" ::: "memory");
-                R v1[6], v2[6];
-                gather(v1, v2);
-                bool in = true;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const bool hi = (o >> a) & 1;
-                    const R t1 = hi ? v1[2 * a + 1] : v1[2 * a], t2 = hi ? v2[2 * a + 1] : v2[2 * a];
-                    in = in && (hi ? in1[2 * a + 1] : in1[2 * a]);
-                    p[a].ord = counts(t1, tc) ? (fom && t1 > t2 ? 2 : 1) : 0;
-                    p[a].t1 = p[a].ord ? t1 - sh : R(0);
-                    p[a].t2 = p[a].ord == 2 ? t2 - sh : R(0);
-                }
-                if (!in || !(p[0].ord | p[1].ord | p[2].ord)) continue;
-                const R T = octant_solve<R>(p[0], p[1], p[2], h[0], h[1], h[2], slown);
-                if (T < best) best = T;
-            }
+            const R t1 = one ? o1 : q1, t2 = one ? o2 : q2;   // a dropped axis' other side does not count
+            p[a].ord = counts(t1) ? (fom && t1 > t2 ? 2 : 1) : 0;
+            p[a].t1 = p[a].ord ? t1 - sh : R(0);
+            p[a].t2 = p[a].ord == 2 ? t2 - sh : R(0);
         }
+        if (!(p[0].ord | p[1].ord | p[2].ord)) continue;
+        unsigned weak;
+        const R T = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
+        if (T < best) best = T;
+        if (first) unsure |= weak & drop;
     }
-    if (SHIFT && best < inf) best = tb + best;
     return best;
+}
+
+// One node update.  gather(a) gives axis a's sides of the stencil (every axis
+// has at least two nodes).  FAST selects the axis-sum octant form; otherwise
+// the reference's leading-axis form in the CPU oracle's operation order.
+// h, ih: spacings and their reciprocals along r, x, z.  free: whether the node
+// is one to update (the value returned for another one is not to be used).
+template <typename R, bool FAST, bool SHIFT, typename G>
+__device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], const R ih[3], R slown, bool free = true)
+{
+    const R inf = Lim<R>::inf();
+    // per axis the lower side (t1, t2) -- the counted one, where one counts --
+    // and the least of the other sides: at or below the node, two count
+    R t1[3], t2[3], other = inf;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const AxisSides<R> g = gather(a);
+        const bool lo = g.l1 <= g.h1;
+        t1[a] = lo ? g.l1 : g.h1;
+        t2[a] = lo ? g.l2 : g.h2;
+        const R o = lo ? g.h1 : g.l1;
+        other = o < other ? o : other;
+    }
+    // an unknown node counts every known neighbour: its value compares as the
+    // largest finite one where equal values count, as inf where they do not
+    const R top = SHIFT ? (tc < inf ? tc : std::numeric_limits<R>::max()) : tc;
+    auto counts = [&](R v) { return SHIFT ? v <= top : v < top; };
+    const R low = t1[0] < t1[1] ? (t1[0] < t1[2] ? t1[0] : t1[2]) : (t1[1] < t1[2] ? t1[1] : t1[2]);
+    const bool known = counts(low);   // some neighbour counts
+    const R sh = SHIFT ? low : R(0);
+    const R s2 = slown * slown;
+    const R h2[3] = { h[0] * h[0], h[1] * h[1], h[2] * h[2] };
+    R kt = R(0);
+    Side<R> p[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        p[a].ord = counts(t1[a]) ? (fom && t1[a] > t2[a] ? 2 : 1) : 0;
+        p[a].t1 = FAST || p[a].ord ? t1[a] - sh : R(0);
+        p[a].t2 = FAST || p[a].ord == 2 ? t2[a] - sh : R(0);
+        kt += R(0x1.2p-38) * ih[a] * ih[a];   // the largest (c / H)^2: 9/4
+    }
+    unsigned weak;
+    R best = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
+    if ((weak || counts(other)) && known && free) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt);
+    if (SHIFT && best < inf) best = sh + best;
+    return known ? best : inf;
 }
 
 // Patch index of launch rank r on an axis of n patches ordered outward from
@@ -702,6 +772,69 @@ __device__ __forceinline__ int centre_rank(int r, int s, int n)
     }
     const int d = r - m;
     return hi > lo ? s + d : s - d;
+}
+
+// The patch of launch rank (rx, rz) of a slot, and the direction its wave
+// arrives from along each axis (fx, fz; 0: none, the patch is upstream of
+// everything on that axis).  True for slots ordered outward from the patch
+// holding their earliest fixed node.
+template <typename R>
+__device__ __forceinline__ bool walk_patch(const ColArgs<R>& a, int slot, int rx, int rz, int* bx, int* bz, int* fx, int* fz)
+{
+    const int f0 = a.flow ? a.flow[2 * slot] : 1, f1 = a.flow ? a.flow[2 * slot + 1] : 1;
+    if (f0 >= FLOW_CENTER) {
+        const int sx = min((f0 - FLOW_CENTER) / a.px, a.npx - 1), sz = min((f1 - FLOW_CENTER) / a.pz, a.npz - 1);
+        *bx = centre_rank(rx, sx, a.npx);
+        *bz = centre_rank(rz, sz, a.npz);
+        *fx = *bx > sx ? 1 : (*bx < sx ? -1 : 0);
+        *fz = *bz > sz ? 1 : (*bz < sz ? -1 : 0);
+        return true;
+    }
+    *fx = f0 < 0 ? -1 : 1;
+    *fz = f1 < 0 ? -1 : 1;
+    *bx = *fx > 0 ? rx : a.npx - 1 - rx;
+    *bz = *fz > 0 ? rz : a.npz - 1 - rz;
+    return false;
+}
+
+// Whether patch column b runs in sweep iter (it or a lateral neighbour
+// changed in the sweep before), and the layers it walks: lo..hi, all of them,
+// or (win: alternating walks with layer ranges) the layers within two of one
+// that changed, in this patch or a lateral neighbour, in the sweep before or
+// so far in this one -- every node outside was relaxed after its inputs last
+// changed, and a change inside the walk carries it on past the window.  Read
+// by every lane alike.
+template <typename R>
+__device__ __forceinline__ bool walk_active(const ColArgs<R>& a, int slot, int b, int bx, int bz, int iter, int snr, int snx,
+                                            int snz, bool win, int* lo, int* hi)
+{
+    const int np = a.npx * a.npz;
+    const int nb[5] = { b, bx > 0 ? b - a.npz : b, bx < a.npx - 1 ? b + a.npz : b, bz > 0 ? b - 1 : b, bz < a.npz - 1 ? b + 1 : b };
+    const int* st = a.stamp + (size_t)slot * np;
+    int m = st[b];
+    for (int j = 1; j < 5; ++j) m = max(m, st[nb[j]]);
+    *lo = 0;
+    *hi = snr - 1;
+    if (__builtin_amdgcn_readfirstlane(m) < iter - 1 || bx * a.px >= snx || bz * a.pz >= snz) return false;
+    if (win) {
+        const unsigned long long* lr = a.lrng + (size_t)slot * np * 2;
+        int l = 0x7fffffff, h = -1;
+        for (int j = 0; j < 5; ++j)
+            for (int par = 0; par < 2; ++par) {
+                const unsigned long long v = __hip_atomic_load(lr + 2 * nb[j] + par, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const int tag = (int)(unsigned)(v >> 32);
+                if (tag == iter || tag == iter - 1) {
+                    l = min(l, (int)((v >> 16) & 0xffff));
+                    h = max(h, (int)(v & 0xffff));
+                }
+            }
+        l = __builtin_amdgcn_readfirstlane(l);
+        h = __builtin_amdgcn_readfirstlane(h);
+        // nothing changed near it: no layer to walk
+        *lo = h < 0 ? snr : max(0, l - 2);
+        *hi = h < 0 ? snr - 1 : min(snr - 1, h + 2);
+    }
+    return true;
 }
 
 template <typename R, int PX, int PZ, bool FAST, bool SHIFT>
@@ -993,20 +1126,21 @@ k_column(ColArgs<R> a)
                     const int ix = x0 + lx, iz = z0 + lz;
                     const int own = (lx + 2) * LZ + lz + 2;
                     const R tc = cur[own];
-                    const bool in1[6] = { ir >= 1, ir + 1 < snr, ix >= 1, ix + 1 < snx, iz >= 1, iz + 1 < snz };
-                    auto gather = [&](R v1[6], R v2[6]) {
-                        // side 0 is the layer above (ir-1), side 1 the one below (ir+1)
-                        v1[0] = down ? b1[pl] : u1[pl]; v2[0] = down ? b2[pl] : u2[pl];
-                        v1[1] = down ? u1[pl] : b1[pl]; v2[1] = down ? u2[pl] : b2[pl];
-                        v1[2] = cur[own - LZ]; v2[2] = cur[own - 2 * LZ];
-                        v1[3] = cur[own + LZ]; v2[3] = cur[own + 2 * LZ];
-                        v1[4] = cur[own - 1]; v2[4] = cur[own - 2];
-                        v1[5] = cur[own + 1]; v2[5] = cur[own + 2];
-                        rst.apply(v1, v2);
+                    auto gather = [&](int ax) {
+                        AxisSides<R> g;
+                        if (ax == 0) {   // the layers above (ir-1) and below (ir+1)
+                            const R p1 = b1[pl], p2 = b2[pl], f1 = u1[pl], f2 = u2[pl];
+                            g = { down ? p1 : f1, down ? p2 : f2, down ? f1 : p1, down ? f2 : p2, ir >= 1, ir + 1 < snr };
+                        } else if (ax == 1) {
+                            g = { cur[own - LZ], cur[own - 2 * LZ], cur[own + LZ], cur[own + 2 * LZ], ix >= 1, ix + 1 < snx };
+                        } else {
+                            g = { cur[own - 1], cur[own - 2], cur[own + 1], cur[own + 2], iz >= 1, iz + 1 < snz };
+                        }
+                        return rst.apply(g, ax);
                     };
                     const R h[3] = { hr, hxl, shz[lx] };
                     const R ih[3] = { ihr, ihx, sihz[lx] };
-                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, in1, h, ih, slown), rq);
+                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown), rq);
                     // every lane has read its stencil before any lane writes (one wavefront)
                     __builtin_amdgcn_wave_barrier();
                     if (nv != tc) {
@@ -1074,6 +1208,289 @@ k_column(ColArgs<R> a)
     }
     const bool blk = __syncthreads_or(anyv);
     if (t == 0 && blk) {
+        st[b] = iter;
+        atomicMax(a.lastchg + slot, iter);
+        atomicOr(a.valchg + slot, 1);
+    }
+}
+
+// The column walk on 8 x 8 patches: k_column's walk with one node per lane,
+// so every pass updates all 64 nodes at once (Jacobi) and nothing but the
+// layer's values needs LDS.  A lane keeps its column's window in registers:
+// the four layers walked before, the layer's own values, the two ahead; the
+// value three ahead, and the next layer's slowness, fixed bits and spacing,
+// are loaded a layer early, so that only the 64 halo values (two nodes deep
+// on four sides, one per lane; no corners: the stencil is a cross) are waited
+// for when a layer is staged.  Halo cells outside the grid hold inf from the
+// start and are never written (their lanes write the spare cells behind).
+// Same passes, same order, same values as k_column.  A layer costs 400 VALU
+// instructions in float32 (565 in k_column<8, 8>, whose per-lane 64-bit
+// addresses, lane masks and LDS window it does without) and 15 passes of 225
+// each in float64, where the 8 + 8 nodes of a patch's longest chain set the
+// time: 1.45 k cycles a pass (2.4).  One float64 source at 201^3: 15.6 -> 4.3
+// ms with the one-octant update; a float32 one at 65^3: 0.91 -> 0.68 ms.
+template <typename R, bool FAST, bool SHIFT>
+__global__ void __launch_bounds__(64)
+k_walk8(ColArgs<R> a)
+{
+    constexpr int P = 8, LZ = P + 5, CELLS = (P + 4) * LZ;   // odd row stride: phi neighbours spread over banks
+    __shared__ R cur[CELLS + 2 * LZ + 1];
+    const int np = a.npx * a.npz;
+    // block -> patch (workgroups go round-robin over the 8 XCDs).  Slots in
+    // their first sweep, as far as they share out evenly, have all their
+    // patches on one XCD each, in launch order, so that what their patches
+    // pass on stays in its L2 (a store reaches a waiting patch in 650 cycles
+    // instead of 980, or 1400 across XCDs: that sweep of 50 sources at 201^3
+    // takes 8.3 ms, against 13.3 with rows of patches spread over the XCDs).
+    // The others come first and are placed as k_column places them, a row of
+    // patches per XCD: behind the first group, their rows would wait for the
+    // XCD that finishes last; in its place, an XCD would hold the slots that
+    // happen to have most patches still moving (second sweep: 3.6 ms, 3.1
+    // spread).
+    const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int nspread = uniform_load(a.act, 0), nlocal = uniform_load(a.act, 1);
+    const int kspread = (nspread * a.npx + 7) / 8 * a.npz;
+    const bool local = k >= kspread;
+    int slot, rank;   // the patch's launch rank in its slot
+    if (local) {
+        slot = (k - kspread) / np * 8 + xcd;
+        if (slot >= nlocal) return;
+        slot += nspread;
+        rank = (k - kspread) % np;
+    } else {
+        const int row = k / a.npz * 8 + xcd;
+        if (row >= nspread * a.npx) return;
+        slot = row / a.npx;
+        rank = row % a.npx * a.npz + k % a.npz;
+    }
+    slot = uniform_load(a.act, 2 + slot);
+    if (!a.slot_on[slot]) return;
+    const int iter = a.iterp ? __hip_atomic_load(a.iterp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.iter;
+    int bx, bz, fx, fz;
+    const bool centred = walk_patch(a, slot, rank / a.npz, rank % a.npz, &bx, &bz, &fx, &fz);
+    const int b = bx * a.npz + bz;
+    int* st = a.stamp + (size_t)slot * np;
+    const bool alt = a.walkalt && a.walkalt[slot];
+    const bool down = a.walkalt ? (alt && !(iter & 1)) : (a.down != 0);
+    int* pg = (a.prog && (!alt || centred) && (a.ordered_until == 0 || iter <= a.ordered_until)) ? a.prog + (size_t)slot * np : nullptr;
+    const int pbase = iter * a.pstride;
+    const int t = threadIdx.x;
+    const int snr = a.sdims ? a.sdims[3 * slot] : a.nnr;
+    const int snx = a.sdims ? a.sdims[3 * slot + 1] : a.nnx;
+    const int snz = a.sdims ? a.sdims[3 * slot + 2] : a.nnz;
+    const bool win = alt && a.lrng;
+    int lo, hi;
+    if (!walk_active(a, slot, b, bx, bz, iter, snr, snx, snz, win, &lo, &hi)) {
+        // an idle patch is finished with every layer of this sweep
+        if (pg && t == 0) walk_store(pg, b, pbase + a.nnr, local);
+        return;
+    }
+    if (t == 0) atomicAdd(a.visits, 1ull);
+    // upstream neighbours along the flow, and the progress last seen of them
+    // (done: none there, or no longer waited for)
+    constexpr int done = 0x7fffffff;
+    const int limit = local ? 4 * a.spin_limit : a.spin_limit;   // a poll of the XCD's own L2 is about four times as fast
+    const bool hasx = pg && fx != 0 && bx - fx >= 0 && bx - fx < a.npx, hasz = pg && fz != 0 && bz - fz >= 0 && bz - fz < a.npz;
+    int seen_x = hasx ? 0 : done, seen_z = hasz ? 0 : done;
+    // lanes 0..31 read the theta neighbour's counter, the others the phi one's
+    const unsigned pgo = t < 32 ? (hasx ? b - fx * a.npz : b) : (hasz ? b - fz : b);
+    const size_t NL = (size_t)a.nnx * a.nnz, N = NL * a.nnr;
+    const R inf = Lim<R>::inf();
+    const int x0 = bx * P, z0 = bz * P, lx = t / P, lz = t % P;
+    const int gx = x0 + lx, gz = z0 + lz;
+    const bool in = gx < snx && gz < snz;
+    const unsigned coff = in ? gx * a.nnz + gz : x0 * a.nnz + z0;   // node within a layer
+    const unsigned hoff = min(gx, snx - 1);
+    const int own = in ? (lx + 2) * LZ + lz + 2 : CELLS + LZ;   // lanes outside the grid use the spare cells
+    int ridx;
+    unsigned roff;
+    {
+        const int side = t >> 4, d = (t >> 3) & 1, e = t & 7;
+        const int hx_ = side == 0 ? 1 - d : side == 1 ? P + 2 + d : 2 + e;
+        const int hz_ = side == 2 ? 1 - d : side == 3 ? P + 2 + d : 2 + e;
+        const int rx = x0 + hx_ - 2, rz = z0 + hz_ - 2;
+        const bool ok = rx >= 0 && rx < snx && rz >= 0 && rz < snz;
+        ridx = ok ? hx_ * LZ + hz_ : CELLS + 2 * LZ;
+        roff = ok ? rx * a.nnz + rz : coff;
+    }
+    for (int e = t; e < CELLS + 2 * LZ + 1; e += 64) cur[e] = inf;
+    // float64 fields carry no reference
+    constexpr bool REF = std::is_same<R, float>::value;
+    const double* rs = REF && a.ref ? a.ref + (size_t)slot * (a.nnr + 2) : nullptr;
+    const bool hasref = rs && rs[0] != 0.0;
+    const double tfloor = hasref ? a.tfloor : 0.0;
+    const R rq = hasref ? (R)a.qscale : R(0);
+    const R ptl = hasref ? (R)a.ptol : R(0);
+    const bool lguess = hasref && a.lguess;
+    bool anyv = false, capped = false;
+    unsigned long long nupd = 0, nvis = 0;
+    const int dn = down ? 1 : -1;
+    const int qs = down ? lo : snr - 1 - hi, qw = down ? hi : snr - 1 - lo;
+    int lastq = -1000, chg_lo = 0x7fffffff, chg_hi = -1;
+    if (pg && t == 0 && qs > 0) walk_store(pg, b, pbase + qs, local);
+    if (qs < snr) {
+        const ptrdiff_t step = (ptrdiff_t)dn * (ptrdiff_t)NL;
+        const int ir0 = down ? qs : snr - 1 - qs;
+        R* Tl = a.T + (size_t)slot * N + (size_t)ir0 * NL;          // the layer walked
+        const uint32_t* fb = a.fixbits + (size_t)slot * ((N + 31) / 32);
+        const R* slo = a.slo + slot * a.geo_n;
+        const R* hxs = a.hx + slot * a.geo_hx;
+        const R* hzs = a.hz + slot * a.geo_hz;
+        const R hr = a.hr, ihr = R(1) / a.hr;
+        // one layer's per-node data besides the times
+        uint32_t fw;
+        R sv, hzv;
+        auto fetch = [&](int ir) {
+            const size_t l = (size_t)ir * NL;
+            const unsigned bit = (unsigned)(l & 31) + coff;
+            fw = lane_load(fb + (l >> 5), bit >> 5) >> (bit & 31);
+            sv = lane_load(slo + l, coff);
+            hzv = lane_load(hzs + (size_t)ir * a.nnx, hoff);
+        };
+        // times j layers along the walk from the one at position q (inf outside the grid)
+        auto ahead = [&](int q, int j) { const R v = lane_load(Tl + (q + j < snr ? j * step : 0), coff); return q + j < snr ? v : inf; };
+        R cv = Tl[coff], n1 = ahead(qs, 1), n2 = ahead(qs, 2);
+        R b1 = qs >= 1 ? Tl[-step + (ptrdiff_t)coff] : inf, b2 = qs >= 2 ? Tl[-2 * step + (ptrdiff_t)coff] : inf;
+        R b3 = qs >= 3 ? Tl[-3 * step + (ptrdiff_t)coff] : inf, b4 = qs >= 4 ? Tl[-4 * step + (ptrdiff_t)coff] : inf;
+        fetch(ir0);
+        // steps of the reference between consecutive layers of the walk, from
+        // two layers back to two ahead (multiples of 2^-20 s under 4 s, so
+        // their float32 sums are exact too); a neighbour's value plus its step
+        // is its time in the node's frame
+        R dm2 = R(0), dm1 = R(0), d0 = R(0), d1 = R(0), rgx = R(0), rgz = R(0);
+        double rtop = 0.0;
+        auto refrow = [&](int q) { return uniform_load(rs, down ? min(q, snr - 1) : max(snr - 1 - q, 0)); };
+        if (REF && rs) {
+            rgx = (R)rs[a.nnr]; rgz = (R)rs[a.nnr + 1];
+            const double r0 = refrow(qs), r1 = refrow(qs + 1);
+            rtop = refrow(qs + 2);
+            if (qs >= 1) dm1 = (R)(r0 - refrow(qs - 1));
+            if (qs >= 2) dm2 = (R)(refrow(qs - 1) - refrow(qs - 2));
+            d0 = (R)(r1 - r0);
+            d1 = (R)(rtop - r1);
+        }
+        for (int q = qs; q < snr; ++q) {
+            if (q > qw && q - lastq > 2) break;
+            const int ir = down ? q : snr - 1 - q;
+            // wait (bounded) until the upstream patches have finished this
+            // layer; progress read earlier that already covers it saves the poll
+            const int need = pbase + q + 1;
+            for (int spins = 0; min(seen_x, seen_z) < need;) {
+                const int v = __hip_atomic_load(pg + pgo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (seen_x != done) seen_x = __builtin_amdgcn_readlane(v, 0);
+                if (seen_z != done) seen_z = __builtin_amdgcn_readlane(v, 32);
+                if (min(seen_x, seen_z) >= need) break;
+                if (++spins > limit) {
+                    if (seen_x < need) seen_x = done;
+                    if (seen_z < need) seen_z = done;
+                    if (a.wlost && t == 0) __hip_atomic_store(a.wlost + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(2);
+            }
+            // the halo: device-coherent loads, another XCD may have written it this sweep
+            const R hv = lane_load_coherent(Tl, roff);
+            const R hxl = uniform_load(hxs, ir);
+            const R slown = sv, hzl = hzv;
+            const bool free = in && !(fw & 1u);
+            // for the next layers
+            const R n3 = ahead(q, 3);
+            fetch(q + 1 < snr ? ir + dn : ir);
+            // layer start: a free node not reached yet begins from the stored
+            // values of the nodes walked before it in its column, extrapolated
+            // by the polynomial through up to a.lguess of them
+            R tc = cv;
+            if (lguess && free && !(cv < inf) && b1 < inf) {
+                const int m = a.lguess < 2 || !(b2 < inf) ? 1 : a.lguess < 3 || !(b3 < inf) ? 2 : a.lguess < 4 || !(b4 < inf) ? 3 : 4;
+                tc = m == 4 ? R(4) * (b1 - b2) - R(2) * (b2 - b3) + (b3 - b4) + b3
+                   : m == 3 ? R(3) * (b1 - b2) + b3
+                   : m == 2 ? b1 + (b1 - b2) : b1;
+            }
+            const unsigned nfree = (unsigned)__popcll(__ballot(free));
+            const R h[3] = { hr, hxl, hzl };
+            const R ih[3] = { ihr, R(1) / hxl, R(1) / hzl };
+            const R p1 = REF ? b1 - dm1 : b1, p2 = REF ? b2 - (dm1 + dm2) : b2;
+            const R f1 = REF ? n1 + d0 : n1, f2 = REF ? n2 + (d0 + d1) : n2;
+            cur[own] = tc;
+            cur[ridx] = hv;
+            __builtin_amdgcn_wave_barrier();
+            // passes until one changes nothing (slots with a reference: moves
+            // no node by more than ptl), as k_column's
+            int npass = 0;
+#pragma unroll 1
+            for (int pass = 0; pass < a.maxpass; ++pass) {
+                auto gather = [&](int ax) {
+                    AxisSides<R> g;
+                    if (ax == 0) {
+                        // which of the two layers is the lower index makes no difference to the octants
+                        g = { p1, p2, f1, f2, q >= 1, q + 1 < snr };
+                    } else if (ax == 1) {
+                        g = { cur[own - LZ], cur[own - 2 * LZ], cur[own + LZ], cur[own + 2 * LZ], gx >= 1, gx + 1 < snx };
+                        if constexpr (REF) { g.l1 -= rgx; g.l2 -= rgx + rgx; g.h1 += rgx; g.h2 += rgx + rgx; }
+                    } else {
+                        g = { cur[own - 1], cur[own - 2], cur[own + 1], cur[own + 2], gz >= 1, gz + 1 < snz };
+                        if constexpr (REF) { g.l1 -= rgz; g.l2 -= rgz + rgz; g.h1 += rgz; g.h2 += rgz + rgz; }
+                    }
+                    return g;
+                };
+                R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown, free), rq);
+                nv = free ? nv : tc;
+                // every lane has read its stencil before any lane writes (one wavefront)
+                __builtin_amdgcn_wave_barrier();
+                const bool moved = nv != tc && !(fabs(nv - tc) <= ptl);
+                cur[own] = nv;
+                tc = nv;
+                __builtin_amdgcn_wave_barrier();
+                ++npass;
+                if (!__ballot(moved)) break;
+                if (pass == a.maxpass - 1) capped = true;
+            }
+            nupd += nfree * (unsigned)npass;
+            nvis += nfree;
+            // write back what changed; the layer becomes the one before
+            if (tc != cv) walk_store(Tl, coff, tc, local);
+            if (win || !anyv) {
+                const bool fin_n = tc < inf, fin_t = cv < inf;
+                const bool c = tc != cv && (fin_n != fin_t ||
+                    !(fabs((double)tc - (double)cv) <= a.tol * fmax(fmax(fabs((double)tc), fabs((double)cv)), tfloor)));
+                if (__ballot(c)) {
+                    anyv = true;
+                    lastq = q;
+                    chg_lo = min(chg_lo, ir);
+                    chg_hi = max(chg_hi, ir);
+                }
+            }
+            b4 = b3; b3 = b2; b2 = b1; b1 = tc;
+            cv = n1; n1 = n2; n2 = n3;
+            if (REF && rs) {
+                const double r = refrow(q + 3);
+                dm2 = dm1; dm1 = d0; d0 = d1;
+                d1 = (R)(r - rtop);
+                rtop = r;
+            }
+            Tl += step;
+            // publish the layer once its stores have completed
+            if (pg) {
+                __builtin_amdgcn_s_waitcnt(0);
+                if (t == 0) walk_store(pg, b, need, local);
+            }
+        }
+    }
+    if (t != 0) return;
+    // layers the walk did not reach are finished too
+    if (pg) walk_store(pg, b, pbase + a.nnr, local);
+    // a layer left short of its fixpoint: the fixed-point check counts the
+    // patch as moving without evaluating it
+    if (capped && a.pend) {
+        a.pend[(size_t)slot * np + b] = 1;
+        a.slotpend[slot] = 1;
+    }
+    if (win && chg_hi >= 0)
+        __hip_atomic_store(a.lrng + ((size_t)slot * np + b) * 2 + (iter & 1), lrng_pack(iter, chg_lo, chg_hi),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (nupd) atomicAdd(a.updates, nupd);
+    if (nvis) atomicAdd(a.nodes, nvis);
+    if (anyv) {
         st[b] = iter;
         atomicMax(a.lastchg + slot, iter);
         atomicOr(a.valchg + slot, 1);
@@ -1162,36 +1579,38 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         for (int ir = 0; ir < snr; ++ir) {
             const size_t c = (size_t)ir * NL + f;
             if (!((fb[c >> 5] >> (c & 31)) & 1u)) {
-                const bool in1[6] = { ir >= 1, ir + 1 < snr, ix >= 1, ix + 1 < snx, iz >= 1, iz + 1 < snz };
                 rst.layer(rs, ir, snr);
-                // side 0 the layer above (ir-1), side 1 the one below (ir+1);
-                // out of the grid reads as inf, as the walk's staging does
-                auto gather = [&](R v1[6], R v2[6]) {
-                    v1[0] = w[1]; v2[0] = w[0];
-                    v1[1] = w[3]; v2[1] = w[4];
-                    v1[2] = ix >= 1 ? T[c - a.nnz] : inf; v2[2] = ix >= 2 ? T[c - 2 * (size_t)a.nnz] : inf;
-                    v1[3] = ix + 1 < snx ? T[c + a.nnz] : inf; v2[3] = ix + 2 < snx ? T[c + 2 * (size_t)a.nnz] : inf;
-                    v1[4] = iz >= 1 ? T[c - 1] : inf; v2[4] = iz >= 2 ? T[c - 2] : inf;
-                    v1[5] = iz + 1 < snz ? T[c + 1] : inf; v2[5] = iz + 2 < snz ? T[c + 2] : inf;
-                    rst.apply(v1, v2);
+                // axis 0: the layers above (ir-1) and below (ir+1); out of the
+                // grid reads as inf, as the walk's staging does
+                auto gather = [&](int ax) {
+                    AxisSides<R> g;
+                    if (ax == 0) {
+                        g = { w[1], w[0], w[3], w[4], ir >= 1, ir + 1 < snr };
+                    } else if (ax == 1) {
+                        g = { ix >= 1 ? T[c - a.nnz] : inf, ix >= 2 ? T[c - 2 * (size_t)a.nnz] : inf,
+                              ix + 1 < snx ? T[c + a.nnz] : inf, ix + 2 < snx ? T[c + 2 * (size_t)a.nnz] : inf, ix >= 1, ix + 1 < snx };
+                    } else {
+                        g = { iz >= 1 ? T[c - 1] : inf, iz >= 2 ? T[c - 2] : inf, iz + 1 < snz ? T[c + 1] : inf,
+                              iz + 2 < snz ? T[c + 2] : inf, iz >= 1, iz + 1 < snz };
+                    }
+                    return rst.apply(g, ax);
                 };
-                R v1[6], v2[6];
-                gather(v1, v2);
                 // the lowest input relaxed after the node, in its frame
-                R lm = down ? fmin(v1[1], v2[1]) : fmin(v1[0], v2[0]);
-                if (late_x[0]) lm = fmin(lm, v1[2]);
-                if (late_x[1]) lm = fmin(lm, v2[2]);
-                if (late_x[2]) lm = fmin(lm, v1[3]);
-                if (late_x[3]) lm = fmin(lm, v2[3]);
-                if (late_z[0]) lm = fmin(lm, v1[4]);
-                if (late_z[1]) lm = fmin(lm, v2[4]);
-                if (late_z[2]) lm = fmin(lm, v1[5]);
-                if (late_z[3]) lm = fmin(lm, v2[5]);
+                const AxisSides<R> gr = gather(0), gx = gather(1), gz = gather(2);
+                R lm = down ? fmin(gr.h1, gr.h2) : fmin(gr.l1, gr.l2);
+                if (late_x[0]) lm = fmin(lm, gx.l1);
+                if (late_x[1]) lm = fmin(lm, gx.l2);
+                if (late_x[2]) lm = fmin(lm, gx.h1);
+                if (late_x[3]) lm = fmin(lm, gx.h2);
+                if (late_z[0]) lm = fmin(lm, gz.l1);
+                if (late_z[1]) lm = fmin(lm, gz.l2);
+                if (late_z[2]) lm = fmin(lm, gz.h1);
+                if (late_z[3]) lm = fmin(lm, gz.h2);
                 if (!vf || lm <= w[2]) {
                     const R hxl = a.hx[slot * a.geo_hx + ir], hzl = a.hz[slot * a.geo_hz + (size_t)ir * a.nnx + ix];
                     const R h[3] = { hr, hxl, hzl };
                     const R ih[3] = { ihr, R(1) / hxl, R(1) / hzl };
-                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, w[2], gather, in1, h, ih, a.slo[slot * a.geo_n + c]), qs);
+                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, w[2], gather, h, ih, a.slo[slot * a.geo_n + c]), qs);
                     if (nv != w[2] && !(fabs(nv - w[2]) <= vtl)) moved = true;
                 }
             }
@@ -1461,19 +1880,19 @@ k_plane(ColArgs<R> a)
                 const bool fixed = (qf[q] >> (c & 31)) & 1u;
                 if (!fixed) {
                     const int ir = down ? w : nr - 1 - w;
-                    // side 0 is layer ir-1, side 1 layer ir+1; the walk reached ir from ir+1 (up) or ir-1 (down)
-                    auto gather = [&](R v1[6], R v2[6]) {
-                        v1[0] = down ? P1 : N1; v2[0] = down ? P2 : N2;
-                        v1[1] = down ? N1 : P1; v2[1] = down ? N2 : P2;
-                        v1[2] = xm1; v2[2] = xm2; v1[3] = xp1; v2[3] = xp2;
-                        v1[4] = zm1; v2[4] = zm2; v1[5] = zp1; v2[5] = zp2;
+                    // axis 0: layers ir-1 and ir+1; the walk reached ir from ir+1 (up) or ir-1 (down).
+                    // The lateral values are in flow order (upstream first): the octants of either
+                    // order are the same.
+                    auto gather = [&](int ax) {
+                        AxisSides<R> g;
+                        if (ax == 0) g = { down ? P1 : N1, down ? P2 : N2, down ? N1 : P1, down ? N2 : P2, ir >= 1, ir + 1 < nr };
+                        else if (ax == 1) g = { xm1, xm2, xp1, xp2, (lf & 1u) != 0, (lf & 4u) != 0 };
+                        else g = { zm1, zm2, zp1, zp2, (lf & 16u) != 0, (lf & 64u) != 0 };
+                        return g;
                     };
-                    bool in1[6] = { ir >= 1, ir + 1 < nr, false, false, false, false };
-                    in1[2] = lf & 1u; in1[3] = lf & 4u;
-                    in1[4] = lf & 16u; in1[5] = lf & 64u;
                     const R h[3] = { hr, qhx[q], qhz[q] };
                     const R ih[3] = { ihr, fast_rcp(qhx[q]), fast_rcp(qhz[q]) };
-                    const R nv = col_update<R, FAST, SHIFT>(a.fom, C0, gather, in1, h, ih, qs[q]);
+                    const R nv = col_update<R, FAST, SHIFT>(a.fom, C0, gather, h, ih, qs[q]);
                     ++nupd;
                     if (nv != C0) {
                         cur = nv;
@@ -2006,6 +2425,7 @@ struct Slots {
     uint32_t* fix = nullptr;
     int* stamp = nullptr;
     int* lastchg = nullptr;
+    int* act = nullptr;    // slots the next sweep walks (k_next_sweep)
     int* on = nullptr;
     double* toff = nullptr;
     // float32 fields: per slot nnr + 2 values -- the vertical reference
@@ -2464,7 +2884,7 @@ static int ctx_setup(fmm3d_ctx* c, int device, fmm3d_ctx** out)
 static void free_slots(Slots& s)
 {
     (void)hipFree(s.T); (void)hipFree(s.P); (void)hipFree(s.fix); (void)hipFree(s.stamp);
-    (void)hipFree(s.lastchg); (void)hipFree(s.on); (void)hipFree(s.toff); (void)hipFree(s.ref);
+    (void)hipFree(s.lastchg); (void)hipFree(s.on); (void)hipFree(s.act); (void)hipFree(s.toff); (void)hipFree(s.ref);
     (void)hipFree(s.valchg); (void)hipFree(s.prog); (void)hipFree(s.flow); (void)hipFree(s.srcpos); (void)hipFree(s.walkalt);
     (void)hipFree(s.pend); (void)hipFree(s.wlost); (void)hipFree(s.slotpend); (void)hipFree(s.born); (void)hipFree(s.lrng);
     s = Slots();
@@ -2592,6 +3012,7 @@ static int ensure_slots(fmm3d_ctx* c, int nsrc, int prec)
     HIPCHK(c, dalloc(&s.stamp, (size_t)nsrc * nbmax * sizeof(int)));
     HIPCHK(c, dalloc(&s.lastchg, nsrc * sizeof(int)));
     HIPCHK(c, dalloc(&s.on, nsrc * sizeof(int)));
+    HIPCHK(c, dalloc(&s.act, ((size_t)nsrc + 2) * sizeof(int)));
     HIPCHK(c, dalloc(&s.toff, nsrc * sizeof(double)));
     HIPCHK(c, dalloc(&s.ref, (size_t)nsrc * (c->g.nnr + 2) * sizeof(double)));
     HIPCHK(c, dalloc(&s.valchg, nsrc * sizeof(int)));
@@ -2892,10 +3313,61 @@ __global__ void k_pack_rows(int nr, int64_t rcap, const int32_t* __restrict__ co
     }
 }
 
-// the next sweep number, for graph replays of a sweep chunk
-__global__ void k_next_iter(int* p)
+// Before a sweep (one block): its number, and the slots it walks -- on, and
+// changed in the sweep before (the others' patches would all return).  act
+// takes how many of them are spread over the XCDs and how many are placed on
+// one each (a multiple of 8 of the slots in their first sweep), then the
+// indices of the former and of the latter.  The sweep is number iter, or
+// (graph replays) step after the one p holds; p, if any, takes the number.
+// born: each slot's first sweep, or null (sweep 1).
+__global__ void __launch_bounds__(256) k_next_sweep(int* p, int step, int iter, int n, const int* __restrict__ on,
+                                                    const int* __restrict__ lastchg, const int* __restrict__ born,
+                                                    int* __restrict__ act)
 {
-    if (threadIdx.x == 0) p[0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    __shared__ int part[2][4];
+    const int t = threadIdx.x, w = t >> 6;
+    const int it = step ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + step : iter;
+    auto walks = [&](int q) { return q < n && on[q] && lastchg[q] >= it - 1; };
+    auto fresh = [&](int q) { return (born ? born[q] : 1) == it; };
+    // per round of 256 slots, the walked fresh ones (kind 1) and others (kind
+    // 0) before thread t's
+    auto count = [&](int q, int kind, int& before, int& all) {
+        const bool a = walks(q) && fresh(q) == (kind != 0);
+        const unsigned long long m = __ballot(a);
+        __syncthreads();
+        if ((t & 63) == 0) part[kind][w] = __popcll(m);
+        __syncthreads();
+        before = __popcll(m & ((1ull << (t & 63)) - 1));
+        for (int j = 0; j < w; ++j) before += part[kind][j];
+        all = part[kind][0] + part[kind][1] + part[kind][2] + part[kind][3];
+        return a;
+    };
+    int nfresh = 0, nold = 0;
+    for (int q0 = 0; q0 < n; q0 += 256) {
+        int before, all;
+        count(q0 + t, 1, before, all);
+        nfresh += all;
+        count(q0 + t, 0, before, all);
+        nold += all;
+    }
+    const int nlocal = nfresh & ~7, nspread = nold + nfresh - nlocal;
+    int f = 0, o = 0;
+    for (int q0 = 0; q0 < n; q0 += 256) {
+        int before, all;
+        if (count(q0 + t, 1, before, all)) {
+            const int i = f + before;   // the first nlocal of them are the local ones
+            act[2 + (i < nlocal ? nspread + i : nold + i - nlocal)] = q0 + t;
+        }
+        f += all;
+        if (count(q0 + t, 0, before, all)) act[2 + o + before] = q0 + t;
+        o += all;
+    }
+    __syncthreads();   // every thread has read the counter
+    if (t == 0) {
+        act[0] = nspread;
+        act[1] = nlocal;
+        if (p) p[0] = it;
+    }
 }
 
 __global__ void k_fill_int(int* p, int n, int v)
@@ -3054,6 +3526,13 @@ static int sweep_kernel(const fmm3d_ctx* c, int k, bool engine)
     return (!engine && k <= c->plane_sweeps) ? 2 : 1;
 }
 
+// Whether k_walk8 walks the columns: one node per lane, and 32-bit byte
+// offsets within a layer.
+template <typename R> static bool column_one_node(const ColArgs<R>& a)
+{
+    return a.px == 8 && a.pz == 8 && (size_t)a.nnx * a.nnz * sizeof(R) <= 0xffffffffu;
+}
+
 template <typename R, bool FAST, bool SHIFT>
 static hipError_t launch_column(fmm3d_ctx* c, const ColArgs<R>& a, int blocks, int kind)
 {
@@ -3065,11 +3544,11 @@ static hipError_t launch_column(fmm3d_ctx* c, const ColArgs<R>& a, int blocks, i
         else k_plane<R, 4, FAST, SHIFT><<<pb, 64, 0, c->stream>>>(a);
         return hipGetLastError();
     }
-    if (c->strategy == 2) {   // the hyperplane strategy's patches are 8 x 8
-        k_column<R, 8, 8, FAST, SHIFT><<<blocks, 64, 0, c->stream>>>(a);
+    const int px = patch_x(c), pz = patch_z(c);   // the hyperplane strategy's patches are 8 x 8
+    if (column_one_node(a)) {
+        k_walk8<R, FAST, SHIFT><<<blocks, 64, 0, c->stream>>>(a);
         return hipGetLastError();
     }
-    const int px = c->col_px, pz = c->col_pz;
 #define FMM3D_COL_CASE(A, B)                                                   \
     if (px == A && pz == B) {                                                  \
         k_column<R, A, B, FAST, SHIFT><<<blocks, 64, 0, c->stream>>>(a);        \
@@ -3162,7 +3641,8 @@ static int column_args(fmm3d_ctx* c, int nslots, int order, ColArgs<R>& a, int& 
         a.geo_hx = (size_t)g.nnr;
         a.geo_hz = (size_t)g.nnr * g.nnx;
     }
-    blocks = 8 * ((nslots * npx + 7) / 8) * npz;   // rows of patches round-robin over 8 XCDs
+    a.act = s.act;
+    blocks = 8 * ((nslots * npx + 7) / 8) * npz;   // rows of patches round-robin over 8 XCDs (8 slots make whole rounds)
     return FMM3D_OK;
 }
 
@@ -3177,7 +3657,7 @@ static bool column_supported(int px, int pz)
 
 // Queue `n` sweeps starting at sweep k.  A full chunk replays a captured
 // hipGraph (captured once per argument set: n column-walk launches, each
-// followed by k_next_iter, the sweep number living in c->d_iter; kernel
+// followed by k_next_sweep, the sweep number living in c->d_iter; kernel
 // nodes only); other counts, and tracing, launch directly.  With timing on,
 // each launch (or the whole replay, shared out evenly) is timed with events.
 // The fixed-point check kernels after a column-walk launch (they act after
@@ -3209,8 +3689,9 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         a.iterp = nullptr;
         for (int j = 0; j < n; ++j) {
             a.iter = k + j;
-            if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j], c->stream));
             const int kd = sweep_kernel(c, k + j, engine);
+            k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
+            if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j], c->stream));
             hipError_t le = launch_column<R, FAST, SHIFT>(c, a, blocks, kd);
             HIPCHK(c, le);
             if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j + 1], c->stream));
@@ -3262,7 +3743,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
             e = launch_column<R, FAST, SHIFT>(c, a, blocks, kind);
             if (e == hipSuccess && kind == 1 && a.verify > 0 && c->walk_alt != 1) e = launch_verify<R, FAST, SHIFT>(c, a);
             if (e == hipSuccess) {
-                k_next_iter<<<1, 64, 0, c->stream>>>(c->d_iter);
+                k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 1, 0, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
                 e = hipGetLastError();
             }
         }
@@ -3278,7 +3759,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         }
         c->g_sig = sig;
     }
-    k_fill_int<<<1, 1, 0, c->stream>>>(c->d_iter, 1, k);
+    k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 0, k, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
     c->stats.kernel_launches += n;
