@@ -553,6 +553,11 @@ template <typename R> struct RefSteps {
     }
 };
 
+// Progress counters per slot (np patches), in cache lines of the slot's own:
+// an XCD's L2 that holds a line written for a slot of its own does not look
+// past it for another slot's counters.
+template <typename I> __host__ __device__ __forceinline__ constexpr I prog_stride(I np) { return (np + 63) / 64 * 64; }
+
 // A layer-range entry: the sweep it belongs to and the layers lo..hi that changed.
 __host__ __device__ __forceinline__ unsigned long long lrng_pack(int sweep, int lo, int hi)
 {
@@ -892,7 +897,7 @@ k_column(ColArgs<R> a)
     const bool alt = a.walkalt && a.walkalt[slot];
     const bool down = a.walkalt ? (alt && !(iter & 1)) : (a.down != 0);
     // alternating walks wait on their upstream patches only when ordered outward from their source
-    int* pg = (a.prog && (!alt || centred) && (a.ordered_until == 0 || iter <= a.ordered_until)) ? a.prog + (size_t)slot * np : nullptr;
+    int* pg = (a.prog && (!alt || centred) && (a.ordered_until == 0 || iter <= a.ordered_until)) ? a.prog + (size_t)slot * prog_stride(np) : nullptr;
     const int pbase = iter * a.pstride;
     const int t = threadIdx.x;
     // this slot's own grid: nodes beyond it read as outside the grid
@@ -1272,7 +1277,7 @@ k_walk8(ColArgs<R> a)
     int* st = a.stamp + (size_t)slot * np;
     const bool alt = a.walkalt && a.walkalt[slot];
     const bool down = a.walkalt ? (alt && !(iter & 1)) : (a.down != 0);
-    int* pg = (a.prog && (!alt || centred) && (a.ordered_until == 0 || iter <= a.ordered_until)) ? a.prog + (size_t)slot * np : nullptr;
+    int* pg = (a.prog && (!alt || centred) && (a.ordered_until == 0 || iter <= a.ordered_until)) ? a.prog + (size_t)slot * prog_stride(np) : nullptr;
     const int pbase = iter * a.pstride;
     const int t = threadIdx.x;
     const int snr = a.sdims ? a.sdims[3 * slot] : a.nnr;
@@ -1448,7 +1453,8 @@ k_walk8(ColArgs<R> a)
             nupd += nfree * (unsigned)npass;
             nvis += nfree;
             // write back what changed; the layer becomes the one before
-            if (tc != cv) walk_store(Tl, coff, tc, local);
+            // (the grid's first and last layers share cache lines with other slots' fields)
+            if (tc != cv) walk_store(Tl, coff, tc, local && ir > 0 && ir < a.nnr - 1);
             if (win || !anyv) {
                 const bool fin_n = tc < inf, fin_t = cv < inf;
                 const bool c = tc != cv && (fin_n != fin_t ||
@@ -1719,7 +1725,7 @@ k_plane(ColArgs<R> a)
     const int b = bx * a.npz + bz;
     int* st = a.stamp + (size_t)slot * np;
     const bool down = a.walkalt ? (alt && !(iter & 1)) : (a.down != 0);
-    int* pg = (a.prog && !alt) ? a.prog + (size_t)slot * np : nullptr;
+    int* pg = (a.prog && !alt) ? a.prog + (size_t)slot * prog_stride(np) : nullptr;
     const int nr = a.nnr, nsteps = nr + 2 * (P - 1);
     const int pbase = iter * a.pstride;
     const int t = threadIdx.x;
@@ -3016,7 +3022,7 @@ static int ensure_slots(fmm3d_ctx* c, int nsrc, int prec)
     HIPCHK(c, dalloc(&s.toff, nsrc * sizeof(double)));
     HIPCHK(c, dalloc(&s.ref, (size_t)nsrc * (c->g.nnr + 2) * sizeof(double)));
     HIPCHK(c, dalloc(&s.valchg, nsrc * sizeof(int)));
-    HIPCHK(c, dalloc(&s.prog, (size_t)nsrc * nbmax * sizeof(int)));
+    HIPCHK(c, dalloc(&s.prog, (size_t)nsrc * prog_stride(nbmax) * sizeof(int)));
     HIPCHK(c, dalloc(&s.flow, (size_t)nsrc * 2 * sizeof(int)));
     HIPCHK(c, dalloc(&s.srcpos, (size_t)nsrc * 3 * sizeof(double)));
     HIPCHK(c, dalloc(&s.walkalt, (size_t)nsrc * sizeof(int)));
@@ -3319,8 +3325,10 @@ __global__ void k_pack_rows(int nr, int64_t rcap, const int32_t* __restrict__ co
 // one each (a multiple of 8 of the slots in their first sweep), then the
 // indices of the former and of the latter.  The sweep is number iter, or
 // (graph replays) step after the one p holds; p, if any, takes the number.
-// born: each slot's first sweep, or null (sweep 1).
-__global__ void __launch_bounds__(256) k_next_sweep(int* p, int step, int iter, int n, const int* __restrict__ on,
+// born: each slot's first sweep, or null (sweep 1).  Slots whose layers are
+// shorter than two cache lines are not placed on one XCD (their fields share
+// lines beyond the first and last layer).
+__global__ void __launch_bounds__(256) k_next_sweep(int* p, int step, int iter, int n, int layer_nodes, const int* __restrict__ on,
                                                     const int* __restrict__ lastchg, const int* __restrict__ born,
                                                     int* __restrict__ act)
 {
@@ -3350,7 +3358,7 @@ __global__ void __launch_bounds__(256) k_next_sweep(int* p, int step, int iter, 
         count(q0 + t, 0, before, all);
         nold += all;
     }
-    const int nlocal = nfresh & ~7, nspread = nold + nfresh - nlocal;
+    const int nlocal = layer_nodes >= 64 ? nfresh & ~7 : 0, nspread = nold + nfresh - nlocal;
     int f = 0, o = 0;
     for (int q0 = 0; q0 < n; q0 += 256) {
         int before, all;
@@ -3690,7 +3698,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         for (int j = 0; j < n; ++j) {
             a.iter = k + j;
             const int kd = sweep_kernel(c, k + j, engine);
-            k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
+            k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
             if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j], c->stream));
             hipError_t le = launch_column<R, FAST, SHIFT>(c, a, blocks, kd);
             HIPCHK(c, le);
@@ -3743,7 +3751,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
             e = launch_column<R, FAST, SHIFT>(c, a, blocks, kind);
             if (e == hipSuccess && kind == 1 && a.verify > 0 && c->walk_alt != 1) e = launch_verify<R, FAST, SHIFT>(c, a);
             if (e == hipSuccess) {
-                k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 1, 0, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
+                k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 1, 0, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
                 e = hipGetLastError();
             }
         }
@@ -3759,7 +3767,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         }
         c->g_sig = sig;
     }
-    k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 0, k, a.nslots, a.slot_on, a.lastchg, a.born, c->sl.act);
+    k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 0, k, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
     c->stats.kernel_launches += n;
@@ -3778,7 +3786,8 @@ static int run_column(fmm3d_ctx* c, int nsrc, int order, int* sweeps_out)
     const int np = a.npx * a.npz;
     const bool ordered = a.prog != nullptr;
     if (ordered) {
-        k_fill_int<<<(nsrc * np + 255) / 256, 256, 0, c->stream>>>(s.prog, nsrc * np, 0);
+        const int npr = nsrc * prog_stride(np);
+        k_fill_int<<<(npr + 255) / 256, 256, 0, c->stream>>>(s.prog, npr, 0);
         HIPCHK(c, hipGetLastError());
     }
     const int maxit = 4 * (g.nnr + g.nnx + g.nnz) + 200;
@@ -5365,7 +5374,7 @@ int fmm3d_engine_open(fmm3d_ctx* c, int cap, int precision, int order)
     k_fill_int<<<(cap + 255) / 256, 256, 0, c->stream>>>(s.on, cap, 0);
     k_fill_int<<<(cap + 255) / 256, 256, 0, c->stream>>>(s.lastchg, cap, 0);
     k_fill_int<<<(cap + 255) / 256, 256, 0, c->stream>>>(s.valchg, cap, 0);
-    k_fill_int<<<(int)((cap * nbmax + 255) / 256), 256, 0, c->stream>>>(s.prog, (int)(cap * nbmax), 0);
+    k_fill_int<<<(int)((cap * prog_stride(nbmax) + 255) / 256), 256, 0, c->stream>>>(s.prog, (int)(cap * prog_stride(nbmax)), 0);
     k_fill_int<<<(int)((cap * nbmax + 255) / 256), 256, 0, c->stream>>>(s.stamp, (int)(cap * nbmax), -1);
     k_fill_real<double><<<(3 * cap + 255) / 256, 256, 0, c->stream>>>(s.srcpos, (size_t)3 * cap, __builtin_nan(""));
     HIPCHK(c, hipGetLastError());
@@ -5453,7 +5462,7 @@ int fmm3d_engine_admit(fmm3d_ctx* c, int slot, const int64_t* node, const double
         }
         // every patch column of the new slot runs in the next sweep
         k_fill_int<<<(np + 255) / 256, 256, 0, c->stream>>>(s.stamp + (size_t)slot * np, np, c->eng_k - 1);
-        k_fill_int<<<(np + 255) / 256, 256, 0, c->stream>>>(s.prog + (size_t)slot * np, np, 0);
+        k_fill_int<<<(np + 255) / 256, 256, 0, c->stream>>>(s.prog + (size_t)slot * prog_stride(np), np, 0);
         k_lrng_init<<<(np + 255) / 256, 256, 0, c->stream>>>(s.lrng + (size_t)slot * np * 2, np, c->eng_k);
         k_fill_int<<<1, 1, 0, c->stream>>>(s.lastchg + slot, 1, c->eng_k);
         k_fill_int<<<1, 1, 0, c->stream>>>(s.walkalt + slot, 1, walkalt ? 1 : 0);
@@ -5483,7 +5492,7 @@ __global__ void k_slot_setup(int slot, int np, int k, int walkalt, int* __restri
     if (i < np) {
         const size_t p = (size_t)slot * np + i;
         stamp[p] = k - 1;
-        prog[p] = 0;
+        prog[(size_t)slot * prog_stride(np) + i] = 0;
         pend[p] = 0;
         lrng[2 * p + ((k - 1) & 1)] = lrng_pack(k - 1, 0, 0xffff);
         lrng[2 * p + (k & 1)] = lrng_pack(-1000, 0, 0);
