@@ -103,16 +103,17 @@ __device__ __forceinline__ R octant_solve(const Side<R>& sr, const Side<R>& sx, 
 // leaves the ones of two or one axis.  h2: squared spacings.  *weak: the axes
 // (bits) whose term is not certain; without any, this solution T is the least
 // over a node's octants when none of its axes has both sides counted.  The
-// other octants' equations leave out some of this one's squared terms ((c T - D) / H)^2, so at T their left
-// sides fall short of s^2 by the terms left out: where every term is above
-// the rounding of the whole sum, their larger roots lie beyond T in the
-// computed values too, and the minimum over the octants is T to the last bit.
-// A term must be positive (c T > D): the terms weighted by c / H sum to half
-// the equation's slope at T, which is then a root and not where the
-// discriminant was clamped.  The sum's rounding is a few units in the last
-// place of sum (c T / H)^2 + s^2 (times are absolute: T carries the other
-// terms); kt >= 2^-40 sum (c / H)^2 and ks = 2^-40 s^2 put the bound at 2^13
-// of them.
+// other octants' equations leave out some of this one's squared terms
+// ((c T - D) / H)^2, so at T their left sides fall short of s^2 by the terms
+// left out: where one of those is above the rounding of the whole sum, their
+// larger roots lie beyond T in the computed values too, and the minimum over
+// the octants is T to the last bit.  That holds for any octant without an axis
+// whose term is certain.  A term must be positive (c T > D): the terms
+// weighted by c / H sum to half the equation's slope at T.  Where the
+// discriminant was clamped T is no root, and no term is certain.  The sum's
+// rounding is a few units in the last place of sum (c T / H)^2 + s^2 (times
+// are absolute: T carries the other terms); kt >= 2^-40 sum (c / H)^2 and
+// ks = 2^-40 s^2 put the bound at 2^13 of them.
 __device__ __forceinline__ double octant_one(const Side<double> p[3], const double h2[3], double s2, double kt,
                                              double ks, unsigned* weak)
 {
@@ -141,11 +142,12 @@ __device__ __forceinline__ double octant_one(const Side<double> p[3], const doub
     const double qb = 2.0 * u2 * (m0 * e0 * H21 + m1 * e1 * H20);
     const double qc = u2 * (e0 * e0 * H21 + e1 * e1 * H20 - s2 * H20 * H21);
     double disc = qb * qb - 4.0 * qa * qc;
-    if (disc < 0.0) disc = 0.0;
+    const bool clamped = disc < 0.0;
+    if (clamped) disc = 0.0;
     const double X = DL + (-qb + sqrt(disc)) / (2.0 * qa);
     const double T = first ? X : third<double>(X);
     const double thr = fma(kt * T, T, ks);
-    unsigned w = 0;
+    unsigned w = clamped ? 7u : 0u;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         // an absent axis compares T^2 itself
