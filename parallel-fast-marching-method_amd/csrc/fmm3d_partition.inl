@@ -434,79 +434,154 @@ __global__ void k_pt_start(PartArgs a)
 
 // ---------------------------------------------------------------- the march as a relaxation
 
-// Pop-order update (see the file comment).  Sides r-, r+, x-, x+, z-, z+:
-// v1/v2 first and second neighbour values (+inf unknown), in1/in2 inside the
-// block; t0 the starting value (+inf unknown).  Second order on a side iff
-// its second neighbour is known and below the first (F:645-707).
-__device__ __forceinline__ double pt_pop_update(int fom, double t0, const double v1[6], const double v2[6],
-                                                const bool in1[6], const bool in2[6], double hr, double hx,
-                                                double hz, double slown)
+// Pop-order update (see the file comment).  gather(a) gives axis a's sides
+// (inf unknown or outside the block, and whether the first neighbours are
+// inside it); t0 the starting value (inf unknown).  Second order on a side iff
+// its second neighbour is known and below the first (F:645-707).  tc, the
+// value so far, only says which sides to expect: the result depends on the
+// neighbours alone.
+//
+// The joins meet every octant of joined sides when the last of its sides
+// joins; an axis is left out of it if one of the axis' sides inside the block
+// has not joined by then.  So take the sides below a guess of the result, and
+// fin, the least of t0 and the solutions of their octants: if all of them are
+// below fin, every one joins, and if every other side is at or above it, none
+// follows, and fin is the result to the last bit.  With one side per axis
+// taken and every term certain (octant_one), no octant of fewer sides is below
+// the octant of all of them: one octant decides.  Otherwise the octants of
+// either side of an axis, and those without an axis whose term is not certain,
+// are evaluated too.  The guesses are the value so far, then the last fin; a
+// node none settles takes the joins one by one.  The solve of eight sources at
+// 31x110x140 takes 124 ms with this and 261 ms with all octants of every join
+// at every node (73 and 181 ms for another model).
+template <typename G>
+__device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G gather, double hr, double hx,
+                                                double hz, const double ih[3], double slown)
 {
     const double inf = __builtin_huge_val();
-    bool sec[6];
-    int rank[6];
+    const double h2[3] = { hr * hr, hx * hx, hz * hz }, s2 = slown * slown;
+    // the largest (c / H)^2: 9/4
+    const double kt = 0x1.2p-38 * (ih[0] * ih[0] + ih[1] * ih[1] + ih[2] * ih[2]), ks = 0x1p-40 * s2;
+    double guess = tc < t0 ? tc : t0;
+    bool ok = false;
+#pragma unroll 1
+    for (int attempt = 0; attempt < 4 && !ok; ++attempt) {
+        Side<double> p[3];
+        double last = -inf, next = inf;   // the latest side taken, the earliest left
+        unsigned taken = 0, both = 0;     // axes with a side taken, with two
 #pragma unroll
-    for (int q = 0; q < 6; ++q) sec[q] = fom && in1[q] && in2[q] && v1[q] < inf && v2[q] < inf && v1[q] > v2[q];
-    // rank of each known side in (value, side) order; unknown sides rank 6
+        for (int a = 0; a < 3; ++a) {
+            const AxisSides<double> g = gather(a);
+            const bool lo = g.l1 <= g.h1;
+            const double t1 = lo ? g.l1 : g.h1, t2 = lo ? g.l2 : g.h2, o = lo ? g.h1 : g.l1;
+            const bool take = t1 < guess, two = o < guess;
+            p[a].ord = take ? (fom && t1 > t2 ? 2 : 1) : 0;
+            p[a].t1 = take ? t1 : 0.0;
+            p[a].t2 = p[a].ord == 2 ? t2 : 0.0;
+            const double left = two ? inf : take ? o : t1, got = two ? o : t1;
+            next = left < next ? left : next;
+            last = take && got > last ? got : last;
+            taken |= take ? 1u << a : 0u;
+            both |= two ? 1u << a : 0u;
+        }
+        unsigned weak;
+        double T = octant_one(p, h2, s2, kt, ks, &weak);
+        double fin = taken && T < t0 ? T : t0;
+        weak &= taken;
+        if (weak | both) {
+            unsigned open = weak;
+#pragma unroll 1
+            for (unsigned m = 1; m < 64; ++m) {
+                // c: the axes whose other side is taken instead, d: the axes left out
+                const unsigned c = m >> 3, d = m & 7;
+                if ((c & ~both) || (c & d) || !(taken & ~d)) { m |= c & ~both ? 7 : 0; continue; }
+                if (d & ~open) continue;
+                Side<double> r[3];
+                double top = -inf;        // the last of this octant's sides to join, and its place
+                int at = -1;
+                bool reached = true;
+                double before[3];         // per axis left out: when its last side inside the block joins
+                asm volatile("" ::: "memory");   // the stencil is read again, not kept
 #pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        int r = 0;
+                for (int a = 0; a < 3; ++a) {
+                    const AxisSides<double> g = gather(a);
+                    const bool lo = g.l1 <= g.h1, other = (c >> a) & 1, out = (d >> a) & 1;
+                    const double o1 = lo ? g.h1 : g.l1, o2 = lo ? g.h2 : g.l2, q1 = lo ? g.l1 : g.h1, q2 = lo ? g.l2 : g.h2;
+                    const double t1 = other ? o1 : q1, t2 = other ? o2 : q2;
+                    const bool use = ((taken >> a) & 1) && !out;
+                    r[a].ord = use ? (fom && t1 > t2 ? 2 : 1) : 0;
+                    r[a].t1 = use ? t1 : 0.0;
+                    r[a].t2 = r[a].ord == 2 ? t2 : 0.0;
+                    if (use && t1 >= top) { top = t1; at = a; }
+                    before[a] = !out ? inf : (lo ? g.hin : g.lin) ? ((both >> a) & 1 ? o1 : inf) : q1;
+                }
 #pragma unroll
-        for (int p = 0; p < 6; ++p)
-            if (p != q) r += (in1[p] && v1[p] < inf && (v1[p] < v1[q] || (v1[p] == v1[q] && p < q))) ? 1 : 0;
-        rank[q] = (in1[q] && v1[q] < inf) ? r : 6;
+                for (int a = 0; a < 3; ++a)
+                    if (before[a] < top || (before[a] == top && a < at)) reached = false;
+                if (!reached) continue;
+                unsigned w;
+                T = octant_one(r, h2, s2, kt, ks, &w);
+                if (T < fin) fin = T;
+                if (d == 0) open = w & taken;   // the terms of the octants without axes of this one
+            }
+        }
+        ok = last < fin && next >= fin;
+        guess = fin;
     }
-    Side<double> sd[3][2];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        sd[q / 2][q % 2].ord = in1[q] ? 0 : -1;
-        sd[q / 2][q % 2].t1 = v1[q];
-        sd[q / 2][q % 2].t2 = v2[q];
-    }
+    if (ok) return guess;
+    // the joins, in (value, side) order
     double cur = t0;
+    unsigned joined = 0;
 #pragma unroll 1
     for (int i = 0; i < 6; ++i) {
         int j = -1;
         double vj = inf;
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
-            if (rank[q] == i) { j = q; vj = v1[q]; }
+        for (int a = 0; a < 3; ++a) {
+            const AxisSides<double> g = gather(a);
+            if (g.l1 < vj && !((joined >> (2 * a)) & 1)) { vj = g.l1; j = 2 * a; }
+            if (g.h1 < vj && !((joined >> (2 * a + 1)) & 1)) { vj = g.h1; j = 2 * a + 1; }
+        }
         if (j < 0 || !(vj < cur)) break;
-#pragma unroll
-        for (int q = 0; q < 6; ++q)
-            if (q == j) sd[q / 2][q % 2].ord = sec[q] ? 2 : 1;
+        joined |= 1u << j;
         // the octants through side j
+#pragma unroll 1
+        for (int o = 0; o < 8; ++o) {
+            if (((o >> (j >> 1)) & 1) != (j & 1)) continue;
+            asm volatile("" ::: "memory");   // the stencil is read again, not kept
+            Side<double> p[3];
+            bool in = true;
 #pragma unroll
-        for (int i0 = 0; i0 < 2; ++i0)
-#pragma unroll
-            for (int i1 = 0; i1 < 2; ++i1)
-#pragma unroll
-                for (int i2 = 0; i2 < 2; ++i2) {
-                    if (j != i0 && j != 2 + i1 && j != 4 + i2) continue;
-                    const Side<double>& s0 = sd[0][i0];
-                    const Side<double>& s1 = sd[1][i1];
-                    const Side<double>& s2 = sd[2][i2];
-                    if (s0.ord < 0 || s1.ord < 0 || s2.ord < 0) continue;
-                    const double Tv = octant_solve<double>(s0, s1, s2, hr, hx, hz, slown);
-                    if (Tv < cur) cur = Tv;
-                }
+            for (int a = 0; a < 3; ++a) {
+                const AxisSides<double> g = gather(a);
+                const bool hi = (o >> a) & 1;
+                const double t1 = hi ? g.h1 : g.l1, t2 = hi ? g.h2 : g.l2;
+                const bool on = (joined >> (2 * a + (hi ? 1 : 0))) & 1;
+                in = in && (hi ? g.hin : g.lin);
+                p[a].ord = on ? (fom && t1 > t2 ? 2 : 1) : 0;
+                p[a].t1 = on ? t1 : 0.0;
+                p[a].t2 = p[a].ord == 2 ? t2 : 0.0;
+            }
+            if (!in) continue;
+            unsigned weak;
+            const double T = octant_one(p, h2, s2, kt, ks, &weak);
+            if (T < cur) cur = T;
+        }
     }
     return cur;
 }
 
 // One sweep of the march relaxation over the marching blocks: a wavefront
 // per (slot, block, 8 x 8 patch column).  Per layer it stages the patch with
-// a two-node ring (inside the block) and relaxes it with Jacobi passes until
-// a pass changes nothing; the two layers walked just before stay in LDS.  A
+// a two-node ring (inside the block; one halo value per lane, no corners) and
+// relaxes it with Jacobi passes until a pass changes nothing; a lane keeps the
+// two layers its column walked just before and the two ahead in registers.  A
 // patch column runs in the first sweep of a pass, or when it or a lateral
 // neighbour changed a value in the sweep before.
 __global__ void __launch_bounds__(64) k_pt_walk(PartArgs a)
 {
-    constexpr int LX = PT_P + 4, LZ = PT_P + 5;
-    __shared__ double cur[LX * LZ];
-    __shared__ double b1[64], b2[64], u1[64], u2[64], t0s[64], sl[64];
-    __shared__ double shz[PT_P];
-    __shared__ int s_act;
+    constexpr int LZ = PT_P + 5, CELLS = (PT_P + 4) * LZ;
+    __shared__ double cur[CELLS + 2 * LZ + 1];
     const int ppb = a.npx * a.npz;
     int w = blockIdx.x;
     const int slot = w / (8 * ppb);
@@ -524,16 +599,14 @@ __global__ void __launch_bounds__(64) k_pt_walk(PartArgs a)
     const bool first = iter == a.pstart[slot];
     int* st = a.stamp + ((size_t)slot * 8 + blk) * ppb;
     const int t = threadIdx.x;
-    if (t == 0) {
+    {
         int m = st[pi];
         if (pxi > 0) m = max(m, st[pi - a.npz]);
         if (pxi < npxb - 1) m = max(m, st[pi + a.npz]);
         if (pzi > 0) m = max(m, st[pi - 1]);
         if (pzi < npzb - 1) m = max(m, st[pi + 1]);
-        s_act = first || m >= iter - 1;
+        if (!first && __builtin_amdgcn_readfirstlane(m) < iter - 1) return;
     }
-    __syncthreads();
-    if (!s_act) return;
     const double inf = __builtin_huge_val();
     const size_t NL = (size_t)a.p.n[1] * a.p.n[2];
     double* T = a.T + (size_t)slot * a.N;
@@ -543,93 +616,84 @@ __global__ void __launch_bounds__(64) k_pt_walk(PartArgs a)
     const int dn = down ? 1 : -1;
     const int x0 = lo[1] + pxi * PT_P, z0 = lo[2] + pzi * PT_P;
     const int xe = lo[1] + len[1], ze = lo[2] + len[2];        // block ends (exclusive)
-    const int r0 = lo[0], re = lo[0] + len[0];
     const int lx = t / PT_P, lz = t % PT_P;
     const int gx = x0 + lx, gz = z0 + lz;
     const bool in = gx < xe && gz < ze;
-    const int own = (lx + 2) * LZ + lz + 2;
+    const size_t coff = in ? (size_t)gx * a.p.n[2] + gz : (size_t)x0 * a.p.n[2] + z0;
+    const int own = in ? (lx + 2) * LZ + lz + 2 : CELLS + LZ;   // lanes outside the block use the spare cells
+    const int hrow = min(gx, xe - 1);
+    int ridx;
+    size_t roff;
+    {
+        const int side = t >> 4, d = (t >> 3) & 1, e = t & 7;
+        const int hx_ = side == 0 ? 1 - d : side == 1 ? PT_P + 2 + d : 2 + e;
+        const int hz_ = side == 2 ? 1 - d : side == 3 ? PT_P + 2 + d : 2 + e;
+        const int rx = x0 + hx_ - 2, rz = z0 + hz_ - 2;
+        const bool ok = rx >= lo[1] && rx < xe && rz >= lo[2] && rz < ze;
+        ridx = ok ? hx_ * LZ + hz_ : CELLS + 2 * LZ;
+        roff = ok ? (size_t)rx * a.p.n[2] + rz : coff;
+    }
+    for (int e = t; e < CELLS + 2 * LZ + 1; e += 64) cur[e] = inf;
+    const bool inx0 = gx - 1 >= lo[1], inx1 = gx + 1 < xe, inz0 = gz - 1 >= lo[2], inz1 = gz + 1 < ze;
     bool anyv = false;
     unsigned long long nupd = 0;
-    for (int q = 0; q < len[0]; ++q) {
-        const int ir = down ? r0 + q : re - 1 - q;
-        const size_t lay = (size_t)ir * NL;
-        const size_t c = lay + (size_t)gx * a.p.n[2] + gz;
-        const double v = in ? T[c] : inf;
-        cur[own] = v;
-        const double orig = v;
-        {
-            const int n1 = ir + dn, n2 = ir + 2 * dn;
-            u1[t] = (in && n1 >= r0 && n1 < re) ? T[c + (ptrdiff_t)dn * (ptrdiff_t)NL] : inf;
-            u2[t] = (in && n2 >= r0 && n2 < re) ? T[c + (ptrdiff_t)(2 * dn) * (ptrdiff_t)NL] : inf;
-            const double s0 = in ? T0[c] : inf;
-            // fixed: alive at the march's start (a known non-heap node at or below the heap minimum)
-            const bool fixed = !in || (s0 > 0.0 && s0 < inf && s0 <= mini);
-            t0s[t] = s0 < 0.0 ? -s0 : s0;
-            sl[t] = fixed ? -1.0 : a.slo[c];
-            if (q == 0) {
-                const int p1 = ir - dn, p2 = ir - 2 * dn;
-                b1[t] = (in && p1 >= r0 && p1 < re) ? T[c - (ptrdiff_t)dn * (ptrdiff_t)NL] : inf;
-                b2[t] = (in && p2 >= r0 && p2 < re) ? T[c - (ptrdiff_t)(2 * dn) * (ptrdiff_t)NL] : inf;
-            }
-        }
+    const ptrdiff_t step = (ptrdiff_t)dn * (ptrdiff_t)NL;
+    int ir = down ? lo[0] : lo[0] + len[0] - 1;
+    size_t lay = (size_t)ir * NL;
+    double b1 = inf, b2 = inf;   // the walk starts at a block face: nothing before it
+    double cv = T[lay + coff], n1 = len[0] > 1 ? T[lay + step + coff] : inf;
+    for (int q = 0; q < len[0]; ++q, ir += dn, lay += step) {
         // lateral ring: neighbouring patches of the same block may be writing it
-        for (int e = t; e < LX * (PT_P + 4); e += 64) {
-            const int hx_ = e / (PT_P + 4), hz_ = e % (PT_P + 4);
-            if (hx_ >= 2 && hx_ < PT_P + 2 && hz_ >= 2 && hz_ < PT_P + 2) continue;
-            const int ggx = x0 + hx_ - 2, ggz = z0 + hz_ - 2;
-            const bool ok = ggx >= lo[1] && ggx < xe && ggz >= lo[2] && ggz < ze;
-            cur[hx_ * LZ + hz_] = ok ? __hip_atomic_load(T + lay + (size_t)ggx * a.p.n[2] + ggz, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT) : inf;
-        }
-        if (t < PT_P) shz[t] = a.hz[(size_t)ir * a.p.n[1] + min(x0 + t, xe - 1)];
+        const double hv = __hip_atomic_load(T + lay + roff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const double n2 = q + 2 < len[0] ? T[lay + 2 * step + coff] : inf;
+        const double s0 = T0[lay + coff];
+        const double slown = a.slo[lay + coff];
+        const double hzl = a.hz[(size_t)ir * a.p.n[1] + hrow];
         const double hxl = a.hx[ir];
-        __syncthreads();
-        const double slown = sl[t];
-        const double t0 = t0s[t];
-        bool in1[6], in2[6];
-        in1[0] = ir - 1 >= r0; in2[0] = ir - 2 >= r0;
-        in1[1] = ir + 1 < re; in2[1] = ir + 2 < re;
-        in1[2] = gx - 1 >= lo[1]; in2[2] = gx - 2 >= lo[1];
-        in1[3] = gx + 1 < xe; in2[3] = gx + 2 < xe;
-        in1[4] = gz - 1 >= lo[2]; in2[4] = gz - 2 >= lo[2];
-        in1[5] = gz + 1 < ze; in2[5] = gz + 2 < ze;
+        // fixed: alive at the march's start (a known non-heap node at or below the heap minimum)
+        const bool free = in && !(s0 > 0.0 && s0 < inf && s0 <= mini);
+        const double t0 = s0 < 0.0 ? -s0 : s0;
+        const double ih[3] = { 1.0 / a.hr, 1.0 / hxl, 1.0 / hzl };
+        const double orig = cv;
+        double tc = cv;
+        cur[own] = tc;
+        cur[ridx] = hv;
+        __builtin_amdgcn_wave_barrier();
         int npass = 0;
 #pragma unroll 1
         for (int pass = 0; pass < a.maxpass; ++pass) {
-            bool moved = false;
-            double nv = 0.0;
-            if (slown >= 0.0) {
-                double v1[6], v2[6];
-                // side 0 is the layer above (ir-1), side 1 the one below (ir+1)
-                v1[0] = down ? b1[t] : u1[t]; v2[0] = down ? b2[t] : u2[t];
-                v1[1] = down ? u1[t] : b1[t]; v2[1] = down ? u2[t] : b2[t];
-                v1[2] = cur[own - LZ]; v2[2] = cur[own - 2 * LZ];
-                v1[3] = cur[own + LZ]; v2[3] = cur[own + 2 * LZ];
-                v1[4] = cur[own - 1]; v2[4] = cur[own - 2];
-                v1[5] = cur[own + 1]; v2[5] = cur[own + 2];
-                nv = pt_pop_update(a.fom, t0, v1, v2, in1, in2, a.hr, hxl, shz[lx], slown);
-                moved = nv != cur[own];
-            }
+            auto gather = [&](int ax) {
+                AxisSides<double> g;
+                if (ax == 0) {   // the layers above (ir-1) and below (ir+1)
+                    const bool ahead = q + 1 < len[0];
+                    g = { down ? b1 : n1, down ? b2 : n2, down ? n1 : b1, down ? n2 : b2, down ? q > 0 : ahead, down ? ahead : q > 0 };
+                } else if (ax == 1) {
+                    g = { cur[own - LZ], cur[own - 2 * LZ], cur[own + LZ], cur[own + 2 * LZ], inx0, inx1 };
+                } else {
+                    g = { cur[own - 1], cur[own - 2], cur[own + 1], cur[own + 2], inz0, inz1 };
+                }
+                return g;
+            };
+            double nv = tc;
+            if (free) nv = pt_pop_update(a.fom, t0, tc, gather, a.hr, hxl, hzl, ih, slown);
             // every lane has read its stencil before any lane writes (one wavefront)
             __builtin_amdgcn_wave_barrier();
-            if (moved) cur[own] = nv;
+            const bool moved = nv != tc;
+            cur[own] = nv;
+            tc = nv;
             __builtin_amdgcn_wave_barrier();
             ++npass;
             if (!__ballot(moved)) break;
         }
         nupd += (unsigned long long)npass;
-        __syncthreads();
-        const double nv = cur[own];
-        const bool lay_chg = in && nv != orig;
-        if (lay_chg) __hip_atomic_store(T + c, nv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        b2[t] = b1[t];
-        b1[t] = nv;
-        anyv |= lay_chg;
-        __syncthreads();
+        if (tc != orig) __hip_atomic_store(T + lay + coff, tc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__ballot(tc != orig)) anyv = true;
+        b2 = b1; b1 = tc;
+        cv = n1; n1 = n2;
     }
-    if (t == 0 && nupd) atomicAdd(a.updates, nupd * (unsigned long long)(min(PT_P, xe - x0) * min(PT_P, ze - z0)));
-    const bool blkchg = __syncthreads_or(anyv);
-    if (t == 0 && blkchg) {
+    if (t != 0) return;
+    if (nupd) atomicAdd(a.updates, nupd * (unsigned long long)(min(PT_P, xe - x0) * min(PT_P, ze - z0)));
+    if (anyv) {
         st[pi] = iter;
         atomicOr(a.chg + slot, 1);
     }
