@@ -22,8 +22,8 @@
 //     value of each in-plane neighbour (first or second) with a smaller key
 //     that is in the heap, the old value of every other; so it can be
 //     computed once those neighbours are done.  One workgroup per
-//     (source, block) runs rounds: every ready node computes from the field
-//     as it stands, then all of them apply.  Key ties go by face index.
+//     (source, block) runs rounds over the nodes the round before made
+//     ready.  Key ties go by face index.
 //   - the march (k_pt_walk): the pop-order update.  The march freezes the
 //     nodes alive at its start and gives every other node the minimum of its
 //     starting value and the octant candidates computed each time a
@@ -89,7 +89,6 @@ struct PartState {
     double* Tprev = nullptr;        // field at the start of the pass (ghosts, change)
     double* T0 = nullptr;           // march start: -value for heap nodes, value otherwise
     uint32_t* hbits = nullptr;      // nodes accepted by this pass's face relaxation (the heap)
-    double* fnew = nullptr;         // face relaxation: per (slot, block) values of a round
     int* on = nullptr;              // per slot: passes continue
     int* dsend = nullptr;           // per slot x block: marched in the previous pass
     int* march = nullptr;           // per slot x block: marches in this pass
@@ -201,7 +200,6 @@ struct PartArgs {
     int* chg;
     int* pstart;
     unsigned long long* err;
-    double* fnew;
     size_t nfmax;
     int npx, npz;          // patches per block per axis (the larger block's)
     int iter;              // sweep number
@@ -218,155 +216,183 @@ __device__ __forceinline__ size_t pt_idx(const PartGeo& p, int r, int x, int z)
 
 // ---------------------------------------------------------------- face relaxation
 
-// One face node's value from ghost face k (F:1100-1400): the ghost side of
-// the face axis always counts (second order iff near ghost > far ghost), the
-// other side of that axis is not used; an in-plane neighbour counts iff known
-// and below the node (or the node unknown), second order iff its second
-// neighbour is known and below it; face updates are mixed order whatever the
-// .in file says (F:197-383).  Neighbours beyond the block are out of bounds.
-__device__ double pt_face_value(const PartArgs& a, const double* __restrict__ T, int k, const int c[3],
-                                const int lo[3], const int len[3], double gn, double gf)
+// One octant of a face node's value from ghost face k (F:1100-1400): the ghost
+// side of the face axis A always counts (second order iff near ghost > far
+// ghost), the other side of that axis is not used; an in-plane neighbour
+// counts iff known and below the node (or the node unknown), second order iff
+// its second neighbour is known and below it; face updates are mixed order
+// whatever the .in file says (F:197-383).  Neighbours beyond the block are out
+// of bounds: inf, as no octant.  so, si: the octant's sides (-1, 1) of the
+// in-plane axes.
+__device__ __forceinline__ double pt_face_octant(const PartArgs& a, const double* __restrict__ P, const double* T, int A,
+                                                 int outer, int inner, int side, int so, int si, const int c[3],
+                                                 const int lo[3], const int len[3])
 {
     const double inf = __builtin_huge_val();
-    const int A = PT_FACE_AXIS[k], gs = PT_FACE_SIDE[k] > 0 ? 1 : 0;
+    const ptrdiff_t NL = (ptrdiff_t)a.p.n[1] * a.p.n[2];
     const size_t me = pt_idx(a.p, c[0], c[1], c[2]);
     const double tc = T[me];
-    Side<double> sd[3][2];
+    bool ok = true;
+    Side<double> sd[3];
+    // the values before any is used: their loads are in flight together
+    double v1[3], v2[3];
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax)
+    for (int ax = 0; ax < 3; ++ax) {
+        const ptrdiff_t st = ax == 0 ? NL : ax == 1 ? (ptrdiff_t)a.p.n[2] : 1;
+        const int d = ax == A ? side : ax == outer ? so : si;
+        const int q1 = c[ax] + d - lo[ax], q2 = c[ax] + 2 * d - lo[ax];
+        const bool in1 = ax == A || (q1 >= 0 && q1 < len[ax]), in2 = ax == A || (q2 >= 0 && q2 < len[ax]);
+        const double* F = ax == A ? P : T;
+        const size_t m1 = in1 ? me + d * st : me, m2 = in2 ? me + 2 * d * st : me;
+        v1[ax] = F[m1];
+        v2[ax] = F[m2];
+        ok = ok && in1;
+        v2[ax] = in2 ? v2[ax] : inf;
+    }
+    const double hx = a.hx[c[0]], hz = a.hz[(size_t)c[0] * a.p.n[1] + c[1]], slown = a.slo[me];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            Side<double>& S = sd[ax][s];
-            S.ord = 0; S.t1 = 0.0; S.t2 = 0.0;
-            if (ax == A) {
-                if (s != gs) { S.ord = -1; continue; }
-                S.t1 = gn;
-                if (gn > gf) { S.ord = 2; S.t2 = gf; } else S.ord = 1;
-                continue;
-            }
-            const int d = s ? 1 : -1;
-            int p1[3] = { c[0], c[1], c[2] }, p2[3] = { c[0], c[1], c[2] };
-            p1[ax] += d; p2[ax] += 2 * d;
-            if (p1[ax] < lo[ax] || p1[ax] >= lo[ax] + len[ax]) { S.ord = -1; continue; }
-            const double v1 = T[pt_idx(a.p, p1[0], p1[1], p1[2])];
-            if (!(v1 < inf && v1 < tc)) continue;
-            S.ord = 1; S.t1 = v1;
-            if (p2[ax] >= lo[ax] && p2[ax] < lo[ax] + len[ax]) {
-                const double v2 = T[pt_idx(a.p, p2[0], p2[1], p2[2])];
-                if (v2 < inf && v1 > v2) { S.ord = 2; S.t2 = v2; }
-            }
+    for (int ax = 0; ax < 3; ++ax) {
+        Side<double>& S = sd[ax];
+        if (ax == A) {   // an unknown ghost enters as 0
+            S.t1 = v1[ax] < inf ? v1[ax] : 0.0;
+            const double gf = v2[ax] < inf ? v2[ax] : 0.0;
+            S.ord = S.t1 > gf ? 2 : 1;
+            S.t2 = S.ord == 2 ? gf : 0.0;
+        } else {
+            const bool cnt = v1[ax] < inf && v1[ax] < tc;
+            S.ord = cnt ? (v1[ax] > v2[ax] ? 2 : 1) : 0;
+            S.t1 = cnt ? v1[ax] : 0.0;
+            S.t2 = S.ord == 2 ? v2[ax] : 0.0;
         }
-    const double hx = a.hx[c[0]], hz = a.hz[(size_t)c[0] * a.p.n[1] + c[1]];
-    return octant_min<double>(sd, a.hr, hx, hz, a.slo[me]);
+    }
+    return ok ? octant_solve<double>(sd[0], sd[1], sd[2], a.hr, hx, hz, slown) : inf;
 }
 
-// Face k of every block whose neighbour across it marched in the previous
-// pass: one workgroup per (slot, block).  Dynamic LDS: a state byte
-// (0 not in the heap, 1 waiting, 2 computed this round, 3 done) and the
-// dependency mask (in-plane heap neighbours of smaller key) per face node.
-__global__ void __launch_bounds__(PT_FACE_THREADS) k_pt_face(PartArgs a, int k)
+// The faces of every block whose neighbour across them marched in the previous
+// pass, one after the other: one workgroup per (slot, block).  In heap order a
+// node reads the new value of its in-plane heap neighbours of smaller key, so
+// it is ready once they are done.  Dynamic LDS: per node the neighbours (bits)
+// it still waits for, the queue of ready nodes in the order they became so,
+// and a bit for the nodes in the heap.  A round takes what the round before
+// made ready, four lanes a node, each one of its octants; of two neighbours
+// one waits for the other, so no round reads a value it writes.  A round of
+// some 25 ready nodes is latency: with every thread looking through its own
+// nodes for ready ones, each wavefront ran the whole update for one or two
+// lanes, and a pass over the eight sources at 31x110x140 took 4840 us in six
+// launches, one a face; 493 this way (a face of 3850 nodes: 160).
+__global__ void __launch_bounds__(PT_FACE_THREADS) k_pt_face(PartArgs a)
 {
-    extern __shared__ unsigned char pt_lds[];
+    extern __shared__ unsigned pt_lds[];
+    __shared__ int cnt[3];   // nodes made ready by the round before, this round, cleared for the next
     const int slot = blockIdx.x >> 3, blk = blockIdx.x & 7;
     if (slot >= a.nslots || !a.on[slot]) return;
     int bc[3];
     pt_coord(blk, bc);
-    const int A = PT_FACE_AXIS[k], side = PT_FACE_SIDE[k];
-    int nc[3] = { bc[0], bc[1], bc[2] };
-    nc[A] += side;
-    if (nc[A] < 0 || nc[A] > 1) return;
-    const int nb = (nc[0] << 2) | (nc[1] << 1) | nc[2];
-    if (!a.dsend[slot * 8 + nb]) return;
     int lo[3], len[3];
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) { lo[ax] = a.p.lo(ax, bc[ax]); len[ax] = a.p.len(ax, bc[ax]); }
-    int outer, inner;
-    pt_face_axes(k, outer, inner);
-    const int no = len[outer], ni = len[inner], nf = no * ni;
-    const int fa = side < 0 ? lo[A] : lo[A] + len[A] - 1;     // the face plane
-    unsigned char* state = pt_lds;
-    unsigned char* dep = pt_lds + a.nfmax;
     double* T = a.T + (size_t)slot * a.N;
     const double* P = a.Tprev + (size_t)slot * a.N;
-    double* fnew = a.fnew + ((size_t)slot * 8 + blk) * a.nfmax;
     uint32_t* hb = a.hbits + (size_t)slot * a.words;
     const double inf = __builtin_huge_val();
     const int t = threadIdx.x;
-    auto node_of = [&](int fi, int plane, int c[3]) {
-        c[A] = plane; c[outer] = lo[outer] + fi / ni; c[inner] = lo[inner] + fi % ni;
-    };
-    auto key_of = [&](int fi) {
-        int c[3];
-        node_of(fi, fa + side, c);
-        const double v = P[pt_idx(a.p, c[0], c[1], c[2])];
-        return v < inf ? v : 0.0;
-    };
-    // the heap of this face: nodes whose near ghost is below them (or unknown nodes)
-    for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
-        int c[3];
-        node_of(fi, fa, c);
-        const double tf = T[pt_idx(a.p, c[0], c[1], c[2])];
-        state[fi] = key_of(fi) < tf ? 1 : 0;
-    }
-    __syncthreads();
-    // dependencies: in-plane heap neighbours (first and second) of smaller (key, index)
-    const int NBo[8] = { -1, 1, -2, 2, 0, 0, 0, 0 }, NBi[8] = { 0, 0, 0, 0, -1, 1, -2, 2 };
-    for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
-        if (!state[fi]) { dep[fi] = 0; continue; }
-        const int io = fi / ni, ii = fi % ni;
-        const double ki = key_of(fi);
-        unsigned m = 0;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int jo = io + NBo[q], ji = ii + NBi[q];
-            if (jo < 0 || jo >= no || ji < 0 || ji >= ni) continue;
-            const int fj = jo * ni + ji;
-            if (!state[fj]) continue;
-            const double kj = key_of(fj);
-            if (kj < ki || (kj == ki && fj < fi)) m |= 1u << q;
-        }
-        dep[fi] = (unsigned char)m;
-    }
-    __syncthreads();
-    for (int round = 0; round <= nf; ++round) {
-        int did = 0;
-        for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
-            if (state[fi] != 1) continue;
-            const int io = fi / ni, ii = fi % ni;
-            const unsigned m = dep[fi];
-            bool ready = true;
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if ((m >> q) & 1u) ready = ready && state[(io + NBo[q]) * ni + ii + NBi[q]] == 3;
-            if (!ready) continue;
-            int c[3], cg[3];
-            node_of(fi, fa, c);
-            node_of(fi, fa + side, cg);
-            const double gn0 = P[pt_idx(a.p, cg[0], cg[1], cg[2])];
-            node_of(fi, fa + 2 * side, cg);
-            const double gf0 = P[pt_idx(a.p, cg[0], cg[1], cg[2])];
-            fnew[fi] = pt_face_value(a, T, k, c, lo, len, gn0 < inf ? gn0 : 0.0, gf0 < inf ? gf0 : 0.0);
-            state[fi] = 2;
-            did = 1;
-        }
-        // every value of the round is computed from the field before it
-        if (!__syncthreads_or(did)) break;
-        for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
-            if (state[fi] != 2) continue;
+    unsigned* dep = pt_lds;                                            // a byte per node
+    unsigned* heap = dep + (a.nfmax + 3) / 4;                          // a bit per node
+    unsigned short* queue = (unsigned short*)(heap + (a.nfmax + 31) / 32);
+    const int NBo[8] = { -1, 1, -2, 2, 0, 0, 0, 0 }, NBi[8] = { 0, 0, 0, 0, -1, 1, -2, 2 };   // q ^ 1: the opposite one
+#pragma unroll 1
+    for (int k = 0; k < 6; ++k) {
+        const int A = PT_FACE_AXIS[k], side = PT_FACE_SIDE[k];
+        const int across = (A == 0 ? bc[0] : A == 1 ? bc[1] : bc[2]) + side;
+        if (across < 0 || across > 1) continue;
+        if (!a.dsend[slot * 8 + (blk ^ (4 >> A))]) continue;
+        int outer, inner;
+        pt_face_axes(k, outer, inner);
+        const int no = outer == 0 ? len[0] : len[1], ni = inner == 1 ? len[1] : len[2], nf = no * ni;
+        const int lA = A == 0 ? lo[0] : A == 1 ? lo[1] : lo[2], nA = A == 0 ? len[0] : A == 1 ? len[1] : len[2];
+        const int fa = side < 0 ? lA : lA + nA - 1;     // the face plane
+        auto node_of = [&](int io, int ii, int plane, int c[3]) {
+            c[0] = A == 0 ? plane : lo[0] + io;                                   // the outer axis, unless the face's
+            c[1] = A == 1 ? plane : lo[1] + (A == 0 ? io : ii);
+            c[2] = A == 2 ? plane : lo[2] + ii;
+        };
+        auto key_of = [&](int io, int ii) {
             int c[3];
-            node_of(fi, fa, c);
-            const size_t q = pt_idx(a.p, c[0], c[1], c[2]);
-            const double old = T[q], best = fnew[fi];
-            // acceptance as F:1378, strict on the down face (F:2817); unknown old accepts
-            const bool acc = (k == 5) ? (old > best || !(old < inf)) : (old >= best || !(old < inf));
-            if (acc) {
-                T[q] = best;
-                atomicOr(hb + (q >> 5), 1u << (q & 31));
+            node_of(io, ii, fa + side, c);
+            const double v = P[pt_idx(a.p, c[0], c[1], c[2])];
+            return v < inf ? v : 0.0;
+        };
+        // the heap of this face: nodes whose near ghost is below them (or unknown nodes)
+        __syncthreads();
+        for (int w = t; w < (nf + 31) / 32; w += PT_FACE_THREADS) heap[w] = 0u;
+        for (int w = t; w < (nf + 3) / 4; w += PT_FACE_THREADS) dep[w] = 0u;
+        if (t < 3) cnt[t] = 0;
+        __syncthreads();
+        for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
+            const int io = fi / ni, ii = fi - io * ni;
+            int c[3];
+            node_of(io, ii, fa, c);
+            if (key_of(io, ii) < T[pt_idx(a.p, c[0], c[1], c[2])]) atomicOr(heap + (fi >> 5), 1u << (fi & 31));
+        }
+        __syncthreads();
+        // what each waits for: in-plane heap neighbours (first and second) of smaller (key, index)
+        for (int fi = t; fi < nf; fi += PT_FACE_THREADS) {
+            if (!((heap[fi >> 5] >> (fi & 31)) & 1u)) continue;
+            const int io = fi / ni, ii = fi - io * ni;
+            const double ki = key_of(io, ii);
+            unsigned m = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int jo = io + NBo[q], ji = ii + NBi[q];
+                if (jo < 0 || jo >= no || ji < 0 || ji >= ni) continue;
+                const int fj = jo * ni + ji;
+                if (!((heap[fj >> 5] >> (fj & 31)) & 1u)) continue;
+                const double kj = key_of(jo, ji);
+                if (kj < ki || (kj == ki && fj < fi)) m |= 1u << q;
             }
-            state[fi] = 3;
+            if (m) atomicOr(dep + (fi >> 2), m << (8 * (fi & 3)));
+            else queue[atomicAdd(cnt, 1)] = (unsigned short)fi;
+        }
+        // every round but the last takes at least one node
+        int head = 0;
+#pragma unroll 1
+        for (int round = 0, at = 0; round <= nf; ++round) {
+            __syncthreads();
+            const int tail = head + cnt[at], nx = at == 2 ? 0 : at + 1;
+            if (head == tail) break;
+            if (t == 0) cnt[nx == 2 ? 0 : nx + 1] = 0;
+            for (int e = head + (t >> 2); e < tail; e += PT_FACE_THREADS / 4) {
+                const int fi = queue[e], io = fi / ni, ii = fi - io * ni;
+                int c[3];
+                node_of(io, ii, fa, c);
+                const size_t me = pt_idx(a.p, c[0], c[1], c[2]);
+                double best = pt_face_octant(a, P, T, A, outer, inner, side, t & 1 ? 1 : -1, t & 2 ? 1 : -1, c, lo, len);
+                const double old = T[me];
+                best = fmin(best, __shfl_xor(best, 1));
+                best = fmin(best, __shfl_xor(best, 2));
+                // acceptance as F:1378, strict on the down face (F:2817); unknown old accepts
+                const bool acc = (k == 5) ? (old > best || !(old < inf)) : (old >= best || !(old < inf));
+                if ((t & 3) == 0 && acc) {
+                    T[me] = best;
+                    atomicOr(hb + (me >> 5), 1u << (me & 31));
+                }
+                // two of the neighbours each: those that wait for this node alone are ready
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int q = (t & 3) + 4 * h;
+                    const int step = (t & 1 ? 1 : -1) * (t & 2 ? 2 : 1);
+                    const int jo = io + (h ? 0 : step), ji = ii + (h ? step : 0);
+                    if (jo < 0 || jo >= no || ji < 0 || ji >= ni) continue;
+                    const int fj = jo * ni + ji, sh = 8 * (fj & 3);
+                    const unsigned bit = 1u << (q ^ 1);
+                    const unsigned was = (atomicAnd(dep + (fj >> 2), ~(bit << sh)) >> sh) & 255u;
+                    if (was == bit) queue[tail + atomicAdd(cnt + nx, 1)] = (unsigned short)fj;
+                }
+            }
+            head = tail;
+            at = nx;
         }
         __threadfence_block();
-        __syncthreads();
     }
 }
 
@@ -777,7 +803,7 @@ static void part_model_changed(PartState* ps)
 static void part_free(PartState* ps)
 {
     if (!ps) return;
-    (void)hipFree(ps->Tprev); (void)hipFree(ps->T0); (void)hipFree(ps->hbits); (void)hipFree(ps->fnew);
+    (void)hipFree(ps->Tprev); (void)hipFree(ps->T0); (void)hipFree(ps->hbits);
     (void)hipFree(ps->on); (void)hipFree(ps->dsend); (void)hipFree(ps->march); (void)hipFree(ps->mini);
     (void)hipFree(ps->stamp); (void)hipFree(ps->chg); (void)hipFree(ps->pstart); (void)hipFree(ps->err);
     (void)hipFree(ps->seed); (void)hipFree(ps->slo); (void)hipFree(ps->hx); (void)hipFree(ps->hz);
@@ -830,10 +856,10 @@ static int part_prepare(fmm3d_ctx* c, int nsrc)
         ps.model = true;
     }
     if (ps.cap < nsrc) {
-        (void)hipFree(ps.Tprev); (void)hipFree(ps.T0); (void)hipFree(ps.hbits); (void)hipFree(ps.fnew);
+        (void)hipFree(ps.Tprev); (void)hipFree(ps.T0); (void)hipFree(ps.hbits);
         (void)hipFree(ps.on); (void)hipFree(ps.dsend); (void)hipFree(ps.march); (void)hipFree(ps.mini);
         (void)hipFree(ps.stamp); (void)hipFree(ps.chg); (void)hipFree(ps.pstart); (void)hipFree(ps.err);
-        ps.Tprev = ps.T0 = nullptr; ps.hbits = nullptr; ps.fnew = nullptr; ps.on = ps.dsend = ps.march = nullptr;
+        ps.Tprev = ps.T0 = nullptr; ps.hbits = nullptr; ps.on = ps.dsend = ps.march = nullptr;
         ps.mini = nullptr; ps.stamp = ps.chg = ps.pstart = nullptr; ps.err = nullptr;
         ps.cap = 0;
         size_t nf = 0;
@@ -843,12 +869,11 @@ static int part_prepare(fmm3d_ctx* c, int nsrc)
             nf = std::max(nf, (size_t)p.len(outer, 0) * p.len(inner, 0));
         }
         ps.nfmax = nf;
-        if (2 * nf > 65536) return fail(c, FMM3D_E_ARG, "partitioned solve: block faces of %zu nodes exceed 32768", nf);
+        if (nf > 32768) return fail(c, FMM3D_E_ARG, "partitioned solve: block faces of %zu nodes exceed 32768", nf);
         const int npx = (p.len(1, 0) + PT_P - 1) / PT_P, npz = (p.len(2, 0) + PT_P - 1) / PT_P;
         HIPCHK(c, dalloc(&ps.Tprev, (size_t)nsrc * N * sizeof(double)));
         HIPCHK(c, dalloc(&ps.T0, (size_t)nsrc * N * sizeof(double)));
         HIPCHK(c, dalloc(&ps.hbits, (size_t)nsrc * words * sizeof(uint32_t)));
-        HIPCHK(c, dalloc(&ps.fnew, (size_t)nsrc * 8 * nf * sizeof(double)));
         HIPCHK(c, dalloc(&ps.on, (size_t)nsrc * sizeof(int)));
         HIPCHK(c, dalloc(&ps.dsend, (size_t)nsrc * 8 * sizeof(int)));
         HIPCHK(c, dalloc(&ps.march, (size_t)nsrc * 8 * sizeof(int)));
@@ -882,7 +907,7 @@ static int part_run(fmm3d_ctx* c, int nsrc, const double* faces, int order)
     a.T = T; a.Tprev = ps.Tprev; a.T0 = ps.T0; a.hbits = ps.hbits; a.slo = ps.slo; a.hx = ps.hx; a.hz = ps.hz;
     a.hr = g.dnr; a.p = p; a.nslots = nsrc; a.fom = order == FMM3D_ORDER_MIXED ? 1 : 0; a.N = N; a.words = words;
     a.on = ps.on; a.dsend = ps.dsend; a.march = ps.march; a.mini = ps.mini; a.stamp = ps.stamp; a.chg = ps.chg;
-    a.pstart = ps.pstart; a.err = ps.err; a.fnew = ps.fnew; a.nfmax = ps.nfmax; a.npx = npx; a.npz = npz;
+    a.pstart = ps.pstart; a.err = ps.err; a.nfmax = ps.nfmax; a.npx = npx; a.npz = npz;
     a.maxpass = 16; a.updates = c->d_visits + 1;
     hipStream_t st = c->stream;
     const int gsz = (int)std::min<size_t>(((size_t)nsrc * N + 255) / 256, 65536);
@@ -942,7 +967,7 @@ static int part_run(fmm3d_ctx* c, int nsrc, const double* faces, int order)
 
     const double tol = (double)1.0e-5f;   // F:6403, a default-real literal
     const int walk_blocks = nsrc * 8 * npx * npz;
-    const size_t face_lds = 2 * ps.nfmax;
+    const size_t face_lds = (ps.nfmax + 3) / 4 * 4 + (ps.nfmax + 31) / 32 * 4 + 2 * ps.nfmax;
     int iter = 1;
     long total_sweeps = 0;
     ps.passes.assign(nsrc, 0);
@@ -950,7 +975,7 @@ static int part_run(fmm3d_ctx* c, int nsrc, const double* faces, int order)
     for (int pass = 0; pass <= max_pass; ++pass) {
         if (pass > 0) {
             k_pt_pass_begin<<<gsz, 256, 0, st>>>(a);
-            for (int k = 0; k < 6; ++k) k_pt_face<<<nsrc * 8, PT_FACE_THREADS, face_lds, st>>>(a, k);
+            k_pt_face<<<nsrc * 8, PT_FACE_THREADS, face_lds, st>>>(a);
             k_pt_mark<<<nsrc * 8, 256, 0, st>>>(a);
         }
         k_pt_start<<<gsz, 256, 0, st>>>(a);
