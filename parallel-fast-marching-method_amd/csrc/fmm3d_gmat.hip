@@ -9,7 +9,7 @@
 // single precision, entry by entry in that order.  Here the CSR is uploaded
 // once; the transpose comes from a stable radix sort of the entries by
 // column (for rows with ascending columns, the order subinv builds); the
-// products run one thread per column (G^T x) or per row (G x / cd), each a
+// products run 16 lanes per column (G^T x) or per row (G x / cd), each a
 // sequential float32 sum in subinv's order without contraction, so they
 // are subinv's numbers.
 #include <hip/hip_runtime.h>
@@ -79,30 +79,62 @@ __global__ void k_gather_t(int64_t nnz, const int32_t* __restrict__ perm, const 
     }
 }
 
-// y(c) = sum over column c of G(r, c) x(r), rows ascending (subinv.f90:612-616)
-__global__ void k_gtx(int64_t ncols, const int64_t* __restrict__ cp, const int32_t* __restrict__ row,
-                      const float* __restrict__ tval, const float* __restrict__ x, float* __restrict__ y)
+// s + p(lane J of the own 16 lanes), for J = 0 .. 15 in order
+template <int J> __device__ __forceinline__ float add16(float s, float p)
 {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncols; c += (int64_t)gridDim.x * blockDim.x) {
-        float s = 0.0f;
-        for (int64_t k = cp[c]; k < cp[c + 1]; ++k) s = s + tval[k] * x[row[k]];
-        y[c] = s;
-    }
+    if constexpr (J > 0) s = add16<J - 1>(s, p);
+    return s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p), 0x150 + J, 0xf, 0xf, false));   // row_newbcast:J
 }
 
-// y(r) = (sum over row r of G(r, c) x(c)) / cd(r), in file order (subinv.f90:759-767)
-__global__ void k_gx(int64_t nrows, const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
-                     const float* __restrict__ val, const float* __restrict__ x, const float* __restrict__ cd,
-                     float* __restrict__ y)
+// y(i) = (sum over list i of val(k) x(idx(k)), in list order) / cd(i): G^T x over
+// the columns, rows ascending (subinv.f90:612-616), G x / cd over the rows, in
+// file order (subinv.f90:759-767).  Sixteen lanes per list: they load and
+// multiply 64 entries side by side, and each then adds the 64 products in
+// order, so only the additions are serial, one instruction for an entry of each
+// of the wavefront's four lists.  (An entry past the end adds +0, which changes
+// no sum: one that starts from +0 is never -0.)  Bound by latency: a list of
+// 250 entries is four rounds of two dependent loads.  15000 x 19683, 3.75M
+// entries, G^T x and G x: one thread per list, its loads a list apart, 594 and
+// 151 us; one wavefront per list, two instructions an entry, 45 each; 23 so.
+__global__ void __launch_bounds__(256) k_ordered_sums(int64_t n, const int64_t* __restrict__ ptr, const int32_t* __restrict__ idx,
+                                                      const float* __restrict__ val, const float* __restrict__ x,
+                                                      const float* __restrict__ cd, float* __restrict__ y)
 {
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < nrows; r += (int64_t)gridDim.x * blockDim.x) {
+    const int l = threadIdx.x & 15;
+    const int64_t step = (int64_t)gridDim.x * 16;
+    // the four lists of a wavefront stay together (i0: its first), so that the broadcasts run with all lanes
+    for (int64_t i0 = blockIdx.x * (int64_t)16 + (threadIdx.x >> 6) * 4; i0 < n; i0 += step) {
+        const int64_t i = i0 + ((threadIdx.x >> 4) & 3);
+        int64_t k = 0, k1 = 0;
+        if (i < n) { k = ptr[i]; k1 = ptr[i + 1]; }
         float s = 0.0f;
-        for (int64_t k = rp[r]; k < rp[r + 1]; ++k) s = s + val[k] * x[col[k]];
-        y[r] = cd ? s / cd[r] : s;
+        int32_t c[4];
+        float v[4];
+        auto fetch = [&](int64_t at) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t e = at + 16 * j + l;
+                const bool in = e < k1;
+                c[j] = in ? idx[e] : -1;
+                v[j] = in ? val[e] : 0.0f;
+            }
+        };
+        fetch(k);
+        while (__ballot(k < k1)) {
+            float p[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) p[j] = c[j] >= 0 ? v[j] * x[c[j]] : 0.0f;
+            k += 64;
+            fetch(k);   // the next entries are on their way during the sum
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s = add16<15>(s, p[j]);
+        }
+        if (l == 0 && i < n) y[i] = cd ? s / cd[i] : s;
     }
 }
 
 int grid_of(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 65536); }
+int lists_grid(int64_t n) { return (int)std::min<int64_t>((n + 15) / 16, 65536); }
 
 }  // namespace
 
@@ -209,7 +241,7 @@ extern "C" int fmm3d_gmat_gtx(fmm3d_gmat* m, const float* x, float* y)
     hipError_t e = hipSetDevice(m->device);
     if (e == hipSuccess && m->nrows) e = hipMemcpyAsync(m->x, x, m->nrows * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess) {
-        k_gtx<<<grid_of(m->ncols), 256, 0, m->stream>>>(m->ncols, m->cp, m->row, m->tval, m->x, m->y);
+        k_ordered_sums<<<lists_grid(m->ncols), 256, 0, m->stream>>>(m->ncols, m->cp, m->row, m->tval, m->x, nullptr, m->y);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(y, m->y, m->ncols * sizeof(float), hipMemcpyDeviceToHost, m->stream);
@@ -225,7 +257,7 @@ extern "C" int fmm3d_gmat_gx(fmm3d_gmat* m, const float* x, const float* cd, flo
     if (e == hipSuccess) e = hipMemcpyAsync(m->x, x, m->ncols * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess && cd && m->nrows) e = hipMemcpyAsync(m->cd, cd, m->nrows * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess && m->nrows) {
-        k_gx<<<grid_of(m->nrows), 256, 0, m->stream>>>(m->nrows, m->rp, m->col, m->val, m->x, cd ? m->cd : nullptr, m->y);
+        k_ordered_sums<<<lists_grid(m->nrows), 256, 0, m->stream>>>(m->nrows, m->rp, m->col, m->val, m->x, cd ? m->cd : nullptr, m->y);
         e = hipGetLastError();
     }
     if (e == hipSuccess && m->nrows) e = hipMemcpyAsync(y, m->y, m->nrows * sizeof(float), hipMemcpyDeviceToHost, m->stream);
