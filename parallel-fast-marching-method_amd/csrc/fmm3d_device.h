@@ -158,6 +158,12 @@ __device__ __forceinline__ double octant_one(const Side<double> p[3], const doub
     return T;
 }
 
+// The subsets of a set of axes (bits), a bit for each.
+__host__ __device__ __forceinline__ unsigned subsets(unsigned axes)
+{
+    return (unsigned)(0xFF5533110F050301ull >> (8 * axes)) & 255u;
+}
+
 // Minimum over the valid octants of a node whose six sides are prepared.
 template <typename R>
 __device__ __forceinline__ R octant_min(const Side<R> s[3][2], R hr, R hx, R hz, R slown)

@@ -482,9 +482,10 @@ __global__ void k_pt_start(PartArgs a)
 // the octant of all of them: one octant decides.  Otherwise the octants of
 // either side of an axis, and those without an axis whose term is not certain,
 // are evaluated too.  The guesses are the value so far, then the last fin; a
-// node none settles takes the joins one by one.  The solve of eight sources at
-// 31x110x140 takes 124 ms with this and 261 ms with all octants of every join
-// at every node (73 and 181 ms for another model).
+// node none settles takes the joins one by one.  (Eight sources at 31x110x140,
+// two models: 261 and 181 ms with all octants of every join at every node, 124
+// and 73 ms with these; with the patches in flow order, 48 and 21 ms where the
+// lanes take the octants that any of them needs, 38 and 16 ms each its own.)
 template <typename G>
 __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G gather, double hr, double hx,
                                                 double hz, const double ih[3], double slown)
@@ -520,13 +521,24 @@ __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G
         double fin = taken && T < t0 ? T : t0;
         weak &= taken;
         if (weak | both) {
+            // todo: the octants left, bit (c, d): c the axes whose other side is
+            // taken instead, d the axes left out; each lane takes its own.  First
+            // those of all taken axes, then the others their weak axes ask for
             unsigned open = weak;
+            unsigned long long todo = 0;
+#pragma unroll
+            for (int c = 1; c < 8; ++c) todo |= (c & ~both) ? 0ull : 1ull << (8 * c);
 #pragma unroll 1
-            for (unsigned m = 1; m < 64; ++m) {
-                // c: the axes whose other side is taken instead, d: the axes left out
-                const unsigned c = m >> 3, d = m & 7;
-                if ((c & ~both) || (c & d) || !(taken & ~d)) { m |= c & ~both ? 7 : 0; continue; }
-                if (d & ~open) continue;
+            for (bool first = true;;) {
+                if (!todo && first) {
+                    first = false;
+#pragma unroll
+                    for (unsigned c = 0; c < 8; ++c)
+                        todo |= (c & ~both) ? 0ull : (unsigned long long)(subsets(open & ~c) & ~(1u | 1u << taken)) << (8 * c);
+                }
+                if (!todo) break;
+                const unsigned m = __ffsll(todo) - 1, c = m >> 3, d = m & 7;
+                todo &= todo - 1;
                 Side<double> r[3];
                 double top = -inf;        // the last of this octant's sides to join, and its place
                 int at = -1;
@@ -553,7 +565,7 @@ __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G
                 unsigned w;
                 T = octant_one(r, h2, s2, kt, ks, &w);
                 if (T < fin) fin = T;
-                if (d == 0) open = w & taken;   // the terms of the octants without axes of this one
+                if (first) open |= w & taken;
             }
         }
         ok = last < fin && next >= fin;
@@ -613,7 +625,7 @@ __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G
 // sweep carries a value through the whole block; the sweeps' order does not
 // change where they settle (eight sources at 31x110x140, two models: 140 and
 // 101 sweeps, 84 and 56 ms without the waits; 55 and 28 sweeps, 48 and 21 ms
-// with them).
+// with them, before each lane took its own octants).
 __global__ void __launch_bounds__(64, 4) k_pt_walk(PartArgs a)
 {
     constexpr int LZ = PT_P + 5, CELLS = (PT_P + 4) * LZ;

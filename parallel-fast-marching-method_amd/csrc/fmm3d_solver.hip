@@ -637,17 +637,21 @@ __device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], cons
     }
 }
 
-// The minimum over the octants of a node whose one octant was not certain
+// The minimum over the octants of a node whose one octant, of solution best,
+// was not certain on the axes weak, or has both sides of an axis counted
 // (sides counted below top, times relative to sh).  Per axis, role 0 is the
 // lower side and role 1 the other: its octants differ where both sides count
 // (both), and where role 1 leaves the axis out while role 0 counts (drop).
-// In float64 the octants of the counted sides come first, then those without
-// one or more of the axes some of them left uncertain (eight float64 plane
-// waves at 31x110x140, first sweep: 5.2 ms with all eight octants there, 3.3
-// with these; float32 at 201^3 was slower, 8.6 against 12.0 ms).  The stencil is gathered again for
+// In float64 the other octants of the counted sides come first, then those
+// without one or more of the axes some of them left uncertain; each lane goes
+// through its own (their sets differ from node to node), so the wavefront takes
+// the most that one node needs (eight plane waves at 31x110x140, a call: 8.1 ms
+// with the set its nodes need together, 4.5 so; the first sweep took 5.2 ms with
+// all eight octants and 3.3 with that set).  The stencil is gathered again for
 // each, so that this path holds few registers.
 template <typename R, bool FAST, bool SHIFT, typename G>
-__device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const R h2[3], const R ih[3], R s2, R kt)
+__device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const R h2[3], const R ih[3], R s2, R kt,
+                                          R one, unsigned weak)
 {
     auto counts = [&](R v) { return SHIFT ? v <= top : v < top; };
     R best = Lim<R>::inf();
@@ -686,34 +690,40 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
         }
         return best;
     }
-    unsigned both = 0, drop = 0, unsure = 0;
-#pragma unroll 1
-    for (int j = 0; j < 16; ++j) {
-        const unsigned m = j & 7;   // role 1 on these axes
-        const bool first = j < 8;   // counted sides only
-        if (j > 0 && !(first ? (m & ~both) == 0 : (m & ~(both | unsure)) == 0 && (m & unsure))) continue;
+    unsigned both = 0, drop = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const AxisSides<R> g = gather(a);
+        const bool lo = g.l1 <= g.h1, ob = counts(lo ? g.h1 : g.l1);
+        both |= ob ? 1u << a : 0u;
+        drop |= !ob && counts(lo ? g.l1 : g.h1) && (lo ? g.hin : g.lin) ? 1u << a : 0u;
+    }
+    best = one;
+    unsigned unsure = weak & drop;
+    // todo: the octants left, a bit for each set of axes in role 1
+    unsigned todo = subsets(both) & ~1u;
+    for (bool first = true;;) {
+        if (!todo && first) { first = false; todo = subsets(both | unsure) & ~subsets(both); }
+        if (!todo) break;
+        const unsigned m = __ffs(todo) - 1;
+        todo &= todo - 1;
         asm volatile("" ::: "memory");
         Side<R> p[3];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const AxisSides<R> g = gather(a);
-            const bool lo = g.l1 <= g.h1, one = (m >> a) & 1;
+            const bool lo = g.l1 <= g.h1, other = (m >> a) & 1;
             const R o1 = lo ? g.h1 : g.l1, o2 = lo ? g.h2 : g.l2, q1 = lo ? g.l1 : g.h1, q2 = lo ? g.l2 : g.h2;
-            const bool ob = counts(o1);
-            if (j == 0) {
-                both |= ob ? 1u << a : 0u;
-                drop |= !ob && counts(q1) && (lo ? g.hin : g.lin) ? 1u << a : 0u;
-            }
-            const R t1 = one ? o1 : q1, t2 = one ? o2 : q2;   // a dropped axis' other side does not count
+            const R t1 = other ? o1 : q1, t2 = other ? o2 : q2;   // a dropped axis' other side does not count
             p[a].ord = counts(t1) ? (fom && t1 > t2 ? 2 : 1) : 0;
             p[a].t1 = p[a].ord ? t1 - sh : R(0);
             p[a].t2 = p[a].ord == 2 ? t2 - sh : R(0);
         }
         if (!(p[0].ord | p[1].ord | p[2].ord)) continue;
-        unsigned weak;
-        const R T = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
+        unsigned w;
+        const R T = octant_eval<R, FAST>(p, h2, ih, s2, kt, &w);
         if (T < best) best = T;
-        if (first) unsure |= weak & drop;
+        if (first) unsure |= w & drop;
     }
     return best;
 }
@@ -759,7 +769,7 @@ __device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], c
     }
     unsigned weak;
     R best = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
-    if ((weak || counts(other)) && known && free) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt);
+    if ((weak || counts(other)) && known && free) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt, best, weak);
     if (SHIFT && best < inf) best = sh + best;
     return known ? best : inf;
 }
