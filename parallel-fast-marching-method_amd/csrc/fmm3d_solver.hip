@@ -621,10 +621,11 @@ __device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], cons
         const R A = paa[0] + (paa[1] + paa[2]), B = pa[0] * pb[0] + (pa[1] * pb[1] + pa[2] * pb[2]);
         const R bb = pbb[1] + pbb[2], C = (pbb[0] - s2) + bb;
         R disc = fused_mul_sub(B, B, A * C);
-        disc = disc > R(0) ? disc : R(0);
+        const bool clamped = !(disc > R(0));   // T is no root then, and no term certain
+        disc = clamped ? R(0) : disc;
         const R T = (B + fast_sqrt(disc)) * fast_rcp(A);
         const R thr = R(0x1.8p-15) * (pbb[0] + bb + s2);
-        unsigned w = 0;
+        unsigned w = clamped ? 7u : 0u;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const R g = fma(pa[a], T, -pb[a]);
@@ -642,54 +643,22 @@ __device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], cons
 // (sides counted below top, times relative to sh).  Per axis, role 0 is the
 // lower side and role 1 the other: its octants differ where both sides count
 // (both), and where role 1 leaves the axis out while role 0 counts (drop).
-// In float64 the other octants of the counted sides come first, then those
-// without one or more of the axes some of them left uncertain; each lane goes
-// through its own (their sets differ from node to node), so the wavefront takes
-// the most that one node needs (eight plane waves at 31x110x140, a call: 8.1 ms
-// with the set its nodes need together, 4.5 so; the first sweep took 5.2 ms with
-// all eight octants and 3.3 with that set).  The stencil is gathered again for
-// each, so that this path holds few registers.
+// The other octants of the counted sides come first, then those without one or
+// more of the axes some of them left uncertain; each lane goes through its own
+// (their sets differ from node to node), so the wavefront takes the most that
+// one node needs (float64, eight plane waves at 31x110x140, a call: 8.1 ms with
+// the set its nodes need together, 4.5 so; the first sweep took 5.2 ms with all
+// eight octants and 3.3 with that set).  Where a node of the wavefront has more
+// than one such axis, float32 takes all eight: they are cheap there side by side
+// (201^3, 50 plane waves / a refined source at 61^3, a call: 21.7 / 26.8 ms with
+// all eight always, 18.7 / 32.5 never, 18.6 / 25.9 so).  The stencil is gathered
+// again for each, so that this path holds few registers.
 template <typename R, bool FAST, bool SHIFT, typename G>
 __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const R h2[3], const R ih[3], R s2, R kt,
                                           R one, unsigned weak)
 {
     auto counts = [&](R v) { return SHIFT ? v <= top : v < top; };
     R best = Lim<R>::inf();
-    if constexpr (FAST) {
-        // an octant is cheap here (a hardware square root and reciprocal):
-        // all eight, one theta side and one phi side at a time.  Per side
-        // (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side carries
-        // a = NaN, and fmin passes over the octants through it
-        struct Coef { R a, b, c; };
-        auto coef = [&](R w1, R w2, bool in, R ihx) {
-            // selects on plain values keep this branch-free
-            const bool cnt = counts(w1), sec = fom && w1 > w2;
-            const R u1 = w1 - sh, u2 = w2 - sh;
-            const R num = sec ? fma(R(-0.5), u2, u1 + u1) : u1;
-            const R al = ihx * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
-            const R be = cnt ? num * ihx : R(0);
-            return Coef{ in ? al * al : R(__builtin_nan("")), al * be, be * be };
-        };
-#pragma unroll 1
-        for (int o = 0; o < 4; ++o) {
-            asm volatile("" ::: "memory");   // the stencil is read again, not kept
-            const AxisSides<R> r = gather(0), x = gather(1), z = gather(2);
-            const bool hx = o & 1, hz = o & 2;
-            const Coef cx = coef(hx ? x.h1 : x.l1, hx ? x.h2 : x.l2, hx ? x.hin : x.lin, ih[1]);
-            const Coef cz = coef(hz ? z.h1 : z.l1, hz ? z.h2 : z.l2, hz ? z.hin : z.lin, ih[2]);
-            const Coef c0 = coef(r.l1, r.l2, r.lin, ih[0]), c1 = coef(r.h1, r.h2, r.hin, ih[0]);
-            const R Axz = cx.a + cz.a, Bxz = cx.b + cz.b, Cxz = cx.c + cz.c;
-            auto octant = [&](const Coef& c) {
-                const R A = c.a + Axz, B = c.b + Bxz, C = (c.c - s2) + Cxz;
-                R disc = fused_mul_sub(B, B, A * C);
-                disc = disc > R(0) ? disc : R(0);
-                best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
-            };
-            octant(c0);
-            octant(c1);
-        }
-        return best;
-    }
     unsigned both = 0, drop = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -698,8 +667,45 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
         both |= ob ? 1u << a : 0u;
         drop |= !ob && counts(lo ? g.l1 : g.h1) && (lo ? g.hin : g.lin) ? 1u << a : 0u;
     }
-    best = one;
     unsigned unsure = weak & drop;
+    if constexpr (FAST) {
+        if (__any(__popc(both | unsure) > 1)) {
+            // an octant is cheap here (a hardware square root and reciprocal):
+            // all eight, one theta side and one phi side at a time.  Per side
+            // (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side carries
+            // a = NaN, and fmin passes over the octants through it
+            struct Coef { R a, b, c; };
+            auto coef = [&](R w1, R w2, bool in, R ihx) {
+                // selects on plain values keep this branch-free
+                const bool cnt = counts(w1), sec = fom && w1 > w2;
+                const R u1 = w1 - sh, u2 = w2 - sh;
+                const R num = sec ? fma(R(-0.5), u2, u1 + u1) : u1;
+                const R al = ihx * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
+                const R be = cnt ? num * ihx : R(0);
+                return Coef{ in ? al * al : R(__builtin_nan("")), al * be, be * be };
+            };
+#pragma unroll 1
+            for (int o = 0; o < 4; ++o) {
+                asm volatile("" ::: "memory");   // the stencil is read again, not kept
+                const AxisSides<R> r = gather(0), x = gather(1), z = gather(2);
+                const bool hx = o & 1, hz = o & 2;
+                const Coef cx = coef(hx ? x.h1 : x.l1, hx ? x.h2 : x.l2, hx ? x.hin : x.lin, ih[1]);
+                const Coef cz = coef(hz ? z.h1 : z.l1, hz ? z.h2 : z.l2, hz ? z.hin : z.lin, ih[2]);
+                const Coef c0 = coef(r.l1, r.l2, r.lin, ih[0]), c1 = coef(r.h1, r.h2, r.hin, ih[0]);
+                const R Axz = cx.a + cz.a, Bxz = cx.b + cz.b, Cxz = cx.c + cz.c;
+                auto octant = [&](const Coef& c) {
+                    const R A = c.a + Axz, B = c.b + Bxz, C = (c.c - s2) + Cxz;
+                    R disc = fused_mul_sub(B, B, A * C);
+                    disc = disc > R(0) ? disc : R(0);
+                    best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
+                };
+                octant(c0);
+                octant(c1);
+            }
+            return best;
+        }
+    }
+    best = one;
     // todo: the octants left, a bit for each set of axes in role 1
     unsigned todo = subsets(both) & ~1u;
     for (bool first = true;;) {
