@@ -49,16 +49,16 @@ BYTES_PER_NODE_VISIT = 12
 # measured HBM bytes per node visit of the same kernel on this workload:
 # rocprofv3 FETCH_SIZE (x2.000) and WRITE_SIZE (x1.000), each scaled by a
 # 1 GiB copy, over the launches of one batch of 50
-# (profiles/k_column_tele201_batch50_traffic.md)
-MEASURED_BYTES_PER_NODE_VISIT = 44.94 + 8.06
+# (profiles/k_walk8_tele201_batch50_traffic.md)
+MEASURED_BYTES_PER_NODE_VISIT = 21.04 + 7.70
 # wave64 VALU instructions per 64 float32 node updates of the column walk,
 # from the rocprofv3 SQ_INSTS_VALU pass over one batch of 50, and the
 # device's wave64 VALU issue rate at the clock that pass measured
-# (GRBM_GUI_ACTIVE per XCD over the launch time, 2.28 GHz): 256 CUs x 4
+# (GRBM_GUI_ACTIVE per XCD over the launch time, 2.22 GHz): 256 CUs x 4
 # SIMDs, one wave64 instruction per 4 cycles of a 16-lane SIMD
-# (profiles/k_column_tele201_batch50_valu.md)
-VALU_PER_64_UPDATES = 338.8
-VALU_WAVE_ISSUE_PER_S = 256 * 4 * 2.281e9 / 4
+# (profiles/k_walk8_tele201_batch50_valu.md)
+VALU_PER_64_UPDATES = 221.1
+VALU_WAVE_ISSUE_PER_S = 256 * 4 * 2.221e9 / 4
 
 
 def parse():
@@ -578,13 +578,13 @@ def main():
         "latency_ms_per_batch": {"p50": round(float(np.percentile(lat, 50)), 2),
                                  "p99": round(float(np.percentile(lat, 99)), 2)},
         "frechet_entries_per_step": nnz // max(a.steps, 1),
-        "roofline": {"kernel": "k_column (float32 column walk, 8x8 patches)", "bound": "hbm",
+        "roofline": {"kernel": "k_walk8 (float32 column walk, 8x8 patches)", "bound": "hbm",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": round(MEASURED_BYTES_PER_NODE_VISIT * nvis / max(launches, 1)),
                      "traffic_source": "extrapolated: HBM bytes per node visit from the rocprofv3 FETCH_SIZE/"
                                        "WRITE_SIZE pass in profiles/ times this run's node visits per launch",
-                     "launch_timing": "HIP events around each k_column launch on the solver's stream, over "
+                     "launch_timing": "HIP events around each k_walk8 launch on the solver's stream, over "
                                       "as many batches again as the timed ones (direct launches)",
                      "avg_launch_ms": round(avg_launch_ms, 4),
                      "node_visits_per_launch": int(nvis / max(launches, 1)),
