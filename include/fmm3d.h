@@ -273,7 +273,8 @@ int fmm3d_get_stats(const fmm3d_ctx *ctx, fmm3d_stats *out);
  *                   point; 0 float64 from the start
  *   "spin_limit"    polls before such a wait is given up (default 20000;
  *                   four times as many where the neighbour's progress is
- *                   in the same XCD's cache)
+ *                   in the same XCD's cache); also of the waits between
+ *                   patches in the reference-partition mode
  *   "check_every"   column walk: sweeps between convergence checks (1..8,
  *                   default 4); at a check, every source whose last sweep
  *                   changed nothing leaves the remaining sweeps

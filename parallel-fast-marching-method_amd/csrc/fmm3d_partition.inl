@@ -534,7 +534,8 @@ __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G
                     first = false;
 #pragma unroll
                     for (unsigned c = 0; c < 8; ++c)
-                        todo |= (c & ~both) ? 0ull : (unsigned long long)(subsets(open & ~c) & ~(1u | 1u << taken)) << (8 * c);
+                        todo |= (c & ~both) ? 0ull
+                                            : (unsigned long long)(subsets(open & ~c) & ~(1u | 1u << taken)) << (8 * c);
                 }
                 if (!todo) break;
                 const unsigned m = __ffsll(todo) - 1, c = m >> 3, d = m & 7;
@@ -857,7 +858,8 @@ static void part_free(PartState* ps)
     if (!ps) return;
     (void)hipFree(ps->Tprev); (void)hipFree(ps->T0); (void)hipFree(ps->hbits);
     (void)hipFree(ps->on); (void)hipFree(ps->dsend); (void)hipFree(ps->march); (void)hipFree(ps->mini);
-    (void)hipFree(ps->stamp); (void)hipFree(ps->prog); (void)hipFree(ps->flow); (void)hipFree(ps->chg); (void)hipFree(ps->pstart); (void)hipFree(ps->err);
+    (void)hipFree(ps->stamp); (void)hipFree(ps->prog); (void)hipFree(ps->flow);
+    (void)hipFree(ps->chg); (void)hipFree(ps->pstart); (void)hipFree(ps->err);
     (void)hipFree(ps->seed); (void)hipFree(ps->slo); (void)hipFree(ps->hx); (void)hipFree(ps->hz);
     (void)hipHostFree(ps->h_chg); (void)hipHostFree(ps->h_err);
     delete ps;
@@ -910,7 +912,8 @@ static int part_prepare(fmm3d_ctx* c, int nsrc)
     if (ps.cap < nsrc) {
         (void)hipFree(ps.Tprev); (void)hipFree(ps.T0); (void)hipFree(ps.hbits);
         (void)hipFree(ps.on); (void)hipFree(ps.dsend); (void)hipFree(ps.march); (void)hipFree(ps.mini);
-        (void)hipFree(ps.stamp); (void)hipFree(ps.prog); (void)hipFree(ps.flow); (void)hipFree(ps.chg); (void)hipFree(ps.pstart); (void)hipFree(ps.err);
+        (void)hipFree(ps.stamp); (void)hipFree(ps.prog); (void)hipFree(ps.flow);
+        (void)hipFree(ps.chg); (void)hipFree(ps.pstart); (void)hipFree(ps.err);
         ps.Tprev = ps.T0 = nullptr; ps.hbits = nullptr; ps.on = ps.dsend = ps.march = nullptr;
         ps.mini = nullptr; ps.stamp = ps.prog = ps.flow = ps.chg = ps.pstart = nullptr; ps.err = nullptr;
         ps.cap = 0;
@@ -960,7 +963,8 @@ static int part_run(fmm3d_ctx* c, int nsrc, const double* faces, int order)
     PartArgs a{};
     a.T = T; a.Tprev = ps.Tprev; a.T0 = ps.T0; a.hbits = ps.hbits; a.slo = ps.slo; a.hx = ps.hx; a.hz = ps.hz;
     a.hr = g.dnr; a.p = p; a.nslots = nsrc; a.fom = order == FMM3D_ORDER_MIXED ? 1 : 0; a.N = N; a.words = words;
-    a.on = ps.on; a.dsend = ps.dsend; a.march = ps.march; a.mini = ps.mini; a.stamp = ps.stamp; a.prog = ps.prog; a.flow = ps.flow; a.spin_limit = c->spin_limit; a.chg = ps.chg;
+    a.on = ps.on; a.dsend = ps.dsend; a.march = ps.march; a.mini = ps.mini; a.stamp = ps.stamp;
+    a.prog = ps.prog; a.flow = ps.flow; a.spin_limit = c->spin_limit; a.chg = ps.chg;
     a.pstart = ps.pstart; a.err = ps.err; a.nfmax = ps.nfmax; a.npx = npx; a.npz = npz;
     a.maxpass = 16; a.updates = c->d_visits + 1;
     hipStream_t st = c->stream;

@@ -233,7 +233,7 @@ extern "C" int fmm3d_slice_velocity(const fmm3d_grid_desc* d, int device, const 
     for (int i = 1; i <= dice2 + 1; ++i) slice_basis((double)(i - 1) / (double)dice2, in.data() + nv + nui + 4 * (i - 1));
     if (hipSetDevice(device) != hipSuccess) return slice_fail(FMM3D_E_DEVICE, "fmm3d_slice_velocity: hipSetDevice failed");
     // One allocation and one upload: a call that dices 201 x 201 nodes by 5
-    // takes 0.77 ms (0.92 with six allocations and four uploads).  The kernels
+    // takes 0.74 ms (0.81 with six allocations and four uploads).  The kernels
     // are 0.05 of it; the 8 MB result on its way into the caller's pageable
     // memory is most of the rest.
     hipStream_t st = nullptr;
