@@ -46,6 +46,7 @@
 #include "../../include/fmm3d.h"
 #include "fmm3d_device.h"
 #include "fmm3d_engine.h"
+#include "fmm3d_look.h"
 
 using namespace fmm3d;
 
@@ -1551,6 +1552,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
     for (size_t i = blockIdx.x; i < (size_t)a.nslots * nb; i += gridDim.x) {
         const int slot = (int)(i / nb);
         const size_t f0 = (i - (size_t)slot * nb) * 256 + (threadIdx.x & ~63u), f = f0 + lane;
+        if (!look_has_columns(f0, NL)) continue;
         // alternating walks (point sources) are never at their fixed point
         // after one sweep: they are not checked
         if (!a.slot_on[slot] || (a.born && a.born[slot] != iter) || (a.walkalt && a.walkalt[slot])) continue;
@@ -1575,11 +1577,10 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         // its own, and lateral neighbours outside its patch, except those in
         // the patch it waited for on that axis -- and only if that input is
         // not above it (the update counts no neighbour above its result).
-        // Nodes with no such input are not evaluated.  late_x/late_z: per
-        // offset -1, -2, +1, +2, whether that input can be one.
+        // Nodes with no such input are not evaluated.
         const bool vf = a.vfilter && (a.born || iter == 1);
         const bool down = a.walkalt ? false : (a.down != 0);
-        bool late_x[4] = { false, false, false, false }, late_z[4] = { false, false, false, false };
+        LookLate late = { { 0, 0 }, { 0, 0 } };
         if (vf && on) {
             int fx = 0, fz = 0;   // the waited-for patch on each axis is at patch index - f (0: none)
             const int pxo = ix / a.px, pzo = iz / a.pz;
@@ -1594,29 +1595,22 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
                     fz = f1 < 0 ? -1 : 1;
                 }
             }
-            const int off[4] = { -1, -2, 1, 2 };
-            for (int k = 0; k < 4; ++k) {
-                const int jx = ix + off[k], jz = iz + off[k];
-                late_x[k] = jx >= 0 && jx < snx && jx / a.px != pxo && !(fx != 0 && jx / a.px == pxo - fx);
-                late_z[k] = jz >= 0 && jz < snz && jz / a.pz != pzo && !(fz != 0 && jz / a.pz == pzo - fz);
-            }
+            late = look_late(ix, iz, snx, snz, a.px, a.pz, fx, fz);
         }
-        // A patch has eight rows at least, so late inputs lie on one side of
-        // the node only.  Per axis its first and second neighbour there: the
-        // node read (its own where that one is not late), the step to this
-        // node's frame (then inf), and whether it is late for any lane.  Nodes
-        // count from two rows before the wave's first column.
+        // Per axis the first and second late neighbour: the node read (its own
+        // where that one is not late), the step to this node's frame (then
+        // inf), and whether it is late for any lane.
         unsigned ox[2], oz[2];
         R sx[2], sz[2];
         bool any_x[2], any_z[2];
-        const unsigned fo = 2u * (unsigned)a.nnz + (on ? (unsigned)lane : 0u);
+        const unsigned fo = look_node(a.nnz, lane, on, 0, 0);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const int dx = late_x[k] ? -1 - k : late_x[2 + k] ? 1 + k : 0, dz = late_z[k] ? -1 - k : late_z[2 + k] ? 1 + k : 0;
+            const int dx = late.dx[k], dz = late.dz[k];
             any_x[k] = __ballot(dx != 0) != 0;
             any_z[k] = __ballot(dz != 0) != 0;
-            ox[k] = fo + (unsigned)(dx * a.nnz);
-            oz[k] = fo + (unsigned)dz;
+            ox[k] = look_node(a.nnz, lane, on, dx, 0);
+            oz[k] = look_node(a.nnz, lane, on, 0, dz);
             sx[k] = dx ? (R)dx * rst.gx : inf;
             sz[k] = dz ? (R)dz * rst.gz : inf;
         }
