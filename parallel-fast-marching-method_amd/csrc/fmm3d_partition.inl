@@ -629,8 +629,9 @@ __device__ __forceinline__ double pt_pop_update(int fom, double t0, double tc, G
 // with them, before each lane took its own octants).
 __global__ void __launch_bounds__(64, 4) k_pt_walk(PartArgs a)
 {
-    constexpr int LZ = PT_P + 5, CELLS = (PT_P + 4) * LZ;
-    __shared__ double cur[CELLS + 2 * LZ + 1];
+    constexpr int LZ = Patch8::LZ;
+    static_assert(PT_P == Patch8::P, "one node per lane");
+    __shared__ double cur[Patch8::SIZE];
     const int ppb = a.npx * a.npz;
     // patch by patch in flow order, over all slots and blocks: the neighbours
     // a patch waits for start before it
@@ -681,20 +682,19 @@ __global__ void __launch_bounds__(64, 4) k_pt_walk(PartArgs a)
     const int gx = x0 + lx, gz = z0 + lz;
     const bool in = gx < xe && gz < ze;
     const size_t coff = in ? (size_t)gx * a.p.n[2] + gz : (size_t)x0 * a.p.n[2] + z0;
-    const int own = in ? (lx + 2) * LZ + lz + 2 : CELLS + LZ;   // lanes outside the block use the spare cells
+    const int own = Patch8::own(lx, lz, in);
     const int hrow = min(gx, xe - 1);
     int ridx;
     size_t roff;
     {
-        const int side = t >> 4, d = (t >> 3) & 1, e = t & 7;
-        const int hx_ = side == 0 ? 1 - d : side == 1 ? PT_P + 2 + d : 2 + e;
-        const int hz_ = side == 2 ? 1 - d : side == 3 ? PT_P + 2 + d : 2 + e;
+        int hx_, hz_;
+        Patch8::halo(t, &hx_, &hz_);
         const int rx = x0 + hx_ - 2, rz = z0 + hz_ - 2;
         const bool ok = rx >= lo[1] && rx < xe && rz >= lo[2] && rz < ze;
-        ridx = ok ? hx_ * LZ + hz_ : CELLS + 2 * LZ;
+        ridx = ok ? Patch8::cell(hx_, hz_) : Patch8::HALO_OUT;
         roff = ok ? (size_t)rx * a.p.n[2] + rz : coff;
     }
-    for (int e = t; e < CELLS + 2 * LZ + 1; e += 64) cur[e] = inf;
+    for (int e = t; e < Patch8::SIZE; e += 64) cur[e] = inf;
     const bool inx0 = gx - 1 >= lo[1], inx1 = gx + 1 < xe, inz0 = gz - 1 >= lo[2], inz1 = gz + 1 < ze;
     bool anyv = false;
     unsigned long long nupd = 0;

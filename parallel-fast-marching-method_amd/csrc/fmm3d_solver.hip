@@ -47,6 +47,7 @@
 #include "fmm3d_device.h"
 #include "fmm3d_engine.h"
 #include "fmm3d_look.h"
+#include "fmm3d_patch8.h"
 
 using namespace fmm3d;
 
@@ -1255,8 +1256,8 @@ template <typename R, bool FAST, bool SHIFT>
 __global__ void __launch_bounds__(64)
 k_walk8(ColArgs<R> a)
 {
-    constexpr int P = 8, LZ = P + 5, CELLS = (P + 4) * LZ;   // odd row stride: phi neighbours spread over banks
-    __shared__ R cur[CELLS + 2 * LZ + 1];
+    constexpr int P = Patch8::P, LZ = Patch8::LZ;
+    __shared__ R cur[Patch8::SIZE];
     const int np = a.npx * a.npz;
     // block -> patch (workgroups go round-robin over the 8 XCDs).  Slots in
     // their first sweep, as far as they share out evenly, have all their
@@ -1323,19 +1324,18 @@ k_walk8(ColArgs<R> a)
     const bool in = gx < snx && gz < snz;
     const unsigned coff = in ? gx * a.nnz + gz : x0 * a.nnz + z0;   // node within a layer
     const unsigned hoff = min(gx, snx - 1);
-    const int own = in ? (lx + 2) * LZ + lz + 2 : CELLS + LZ;   // lanes outside the grid use the spare cells
+    const int own = Patch8::own(lx, lz, in);
     int ridx;
     unsigned roff;
     {
-        const int side = t >> 4, d = (t >> 3) & 1, e = t & 7;
-        const int hx_ = side == 0 ? 1 - d : side == 1 ? P + 2 + d : 2 + e;
-        const int hz_ = side == 2 ? 1 - d : side == 3 ? P + 2 + d : 2 + e;
+        int hx_, hz_;
+        Patch8::halo(t, &hx_, &hz_);
         const int rx = x0 + hx_ - 2, rz = z0 + hz_ - 2;
         const bool ok = rx >= 0 && rx < snx && rz >= 0 && rz < snz;
-        ridx = ok ? hx_ * LZ + hz_ : CELLS + 2 * LZ;
+        ridx = ok ? Patch8::cell(hx_, hz_) : Patch8::HALO_OUT;
         roff = ok ? rx * a.nnz + rz : coff;
     }
-    for (int e = t; e < CELLS + 2 * LZ + 1; e += 64) cur[e] = inf;
+    for (int e = t; e < Patch8::SIZE; e += 64) cur[e] = inf;
     // float64 fields carry no reference
     constexpr bool REF = std::is_same<R, float>::value;
     const double* rs = REF && a.ref ? a.ref + (size_t)slot * (a.nnr + 2) : nullptr;
