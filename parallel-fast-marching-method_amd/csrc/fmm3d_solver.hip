@@ -1410,6 +1410,7 @@ k_walk8(ColArgs<R> a)
                 }
                 __builtin_amdgcn_s_sleep(2);
             }
+            asm volatile("" ::: "memory");   // what follows is read after the wait
             // the halo: device-coherent loads, another XCD may have written it this sweep
             const R hv = lane_load_coherent(Tl, roff);
             const R hxl = uniform_load(hxs, ir);
