@@ -275,6 +275,10 @@ int fmm3d_get_stats(const fmm3d_ctx *ctx, fmm3d_stats *out);
  *                   four times as many where the neighbour's progress is
  *                   in the same XCD's cache); also of the waits between
  *                   patches in the reference-partition mode
+ *   "placement_skew" column walk: XCDs between consecutive patches of a
+ *                   source whose first sweep is meant for one XCD (0..7,
+ *                   default 0); other values show that a placement that
+ *                   does not hold changes no result
  *   "check_every"   column walk: sweeps between convergence checks (1..8,
  *                   default 4); at a check, every source whose last sweep
  *                   changed nothing leaves the remaining sweeps

@@ -440,7 +440,8 @@ template <typename R> struct ColArgs {
     float qscale;           // slots with a reference: updated values are rounded to multiples of 1/qscale (0: not)
     float ptol;             // slots with a reference: a layer's passes stop after one that moves no node by
                             // more (s), and the fixed-point check counts only such moves (0: exact)
-    int* wlost;             // per slot: a wait on a neighbour was given up in a sweep
+    int* wlost;             // per slot: WALK_LOST once a sweep was not in order; the home of its patches (k_walk8)
+    int skew;               // k_walk8: consecutive patches of a slot placed on one XCD lie this many XCDs apart
     int lguess;             // slots with a reference: a node not yet reached starts its layer's passes
                             // from the polynomial through the lguess nodes walked just before it in its
                             // column (1: the node before; up to 4: the cubic), 0: from infinity
@@ -502,6 +503,22 @@ template <typename P> __device__ __forceinline__ void walk_store(P* p, unsigned 
     P* q = (P*)((char*)p + i * (unsigned)sizeof(P));
     if (local) __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     else __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// What a.wlost keeps of a slot since its reset: whether some patch of it may
+// have read a neighbour out of order (WALK_LOST), and the XCD its patches run
+// on in a sweep that places them on one (the first to report names it).
+// Called by one lane of a patch: a patch on another XCD than the named one
+// makes the slot lost, since values and progress counters that patches pass on
+// through one XCD's L2 reach another's in no particular order.
+constexpr int WALK_LOST = 1;
+__device__ __forceinline__ void walk_home(int* p)
+{
+    const int home = 2 + 2 * (int)(__builtin_amdgcn_s_getreg(3 << 11 | 20) & 15);   // XCC_ID, bits 0-3
+    int seen = 0;
+    if (!__hip_atomic_compare_exchange_strong(p, &seen, home, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &&
+        (seen & ~WALK_LOST) != home)
+        __hip_atomic_fetch_or(p, WALK_LOST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Steps of a slot's reference from node (ir, ix, iz) to its stencil
@@ -1040,7 +1057,7 @@ k_column(ColArgs<R> a)
                     if (++spins > a.spin_limit) {
                         if (seen_x < need) wx = false;
                         if (seen_z < need) wz = false;
-                        if (a.wlost) __hip_atomic_store(a.wlost + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (a.wlost) __hip_atomic_fetch_or(a.wlost + slot, WALK_LOST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         break;
                     }
                     __builtin_amdgcn_s_sleep(2);
@@ -1269,17 +1286,23 @@ k_walk8(ColArgs<R> a)
     // patches per XCD: behind the first group, their rows would wait for the
     // XCD that finishes last; in its place, an XCD would hold the slots that
     // happen to have most patches still moving (second sweep: 3.6 ms, 3.1
-    // spread).
+    // spread).  That block i runs on XCD i mod 8 is how workgroups are handed
+    // out, not something the language promises, so each patch compares the XCD
+    // it ran on with the slot's first (walk_home, at the end).  On another one
+    // it may have read values that were still in the writer's L2, which costs
+    // order but no value: waits are bounded, the end of the kernel makes every
+    // store visible, and the fixed-point check then trusts no neighbour of the
+    // slot to have been waited for.
     const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
     const int nspread = uniform_load(a.act, 0), nlocal = uniform_load(a.act, 1);
     const int kspread = (nspread * a.npx + 7) / 8 * a.npz;
     const bool local = k >= kspread;
     int slot, rank;   // the patch's launch rank in its slot
     if (local) {
-        slot = (k - kspread) / np * 8 + xcd;
+        rank = (k - kspread) % np;
+        slot = (k - kspread) / np * 8 + ((xcd + a.skew * rank) & 7);
         if (slot >= nlocal) return;
         slot += nspread;
-        rank = (k - kspread) % np;
     } else {
         const int row = k / a.npz * 8 + xcd;
         if (row >= nspread * a.npx) return;
@@ -1405,7 +1428,7 @@ k_walk8(ColArgs<R> a)
                 if (++spins > limit) {
                     if (seen_x < need) seen_x = done;
                     if (seen_z < need) seen_z = done;
-                    if (a.wlost && t == 0) __hip_atomic_store(a.wlost + slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (a.wlost && t == 0) __hip_atomic_fetch_or(a.wlost + slot, WALK_LOST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     break;
                 }
                 __builtin_amdgcn_s_sleep(2);
@@ -1503,6 +1526,7 @@ k_walk8(ColArgs<R> a)
     if (t != 0) return;
     // layers the walk did not reach are finished too
     if (pg) walk_store(pg, b, pbase + a.nnr, local);
+    if (local && a.wlost) walk_home(a.wlost + slot);
     // a layer left short of its fixpoint: the fixed-point check counts the
     // patch as moving without evaluating it
     if (capped && a.pend) {
@@ -1585,7 +1609,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         if (vf && on) {
             int fx = 0, fz = 0;   // the waited-for patch on each axis is at patch index - f (0: none)
             const int pxo = ix / a.px, pzo = iz / a.pz;
-            if (a.prog && (a.ordered_until == 0 || iter <= a.ordered_until) && !a.wlost[slot]) {
+            if (a.prog && (a.ordered_until == 0 || iter <= a.ordered_until) && !(a.wlost[slot] & WALK_LOST)) {
                 const int f0 = a.flow ? a.flow[2 * slot] : 1, f1 = a.flow ? a.flow[2 * slot + 1] : 1;
                 if (f0 >= FLOW_CENTER) {
                     const int sx = min((f0 - FLOW_CENTER) / a.px, a.npx - 1), sz = min((f1 - FLOW_CENTER) / a.pz, a.npz - 1);
@@ -2662,6 +2686,7 @@ struct fmm3d_ctx {
     std::vector<float> eng_hout;
     int ordered = 1;               // column walk: patches wait for their upstream neighbours
     int spin_limit = 20000;        // polls (~64 cycles each) before such a wait is given up
+    int placement_skew = 0;        // XCDs between consecutive patches of a slot meant to lie on one (tests)
     int max_sweeps = 0;            // column walk: stop after this many sweeps (0: at convergence)
     bool walk_settled = true;      // the last column-walk solve ended at its fixed point (not at max_sweeps)
     int point_order = 1;           // alternating walks: patches outward from the earliest fixed node, waiting on their inner neighbours
@@ -3692,6 +3717,7 @@ static int column_args(fmm3d_ctx* c, int nslots, int order, ColArgs<R>& a, int& 
     a.walkalt = s.walkalt;
     a.flow = s.flow;
     a.spin_limit = c->spin_limit;
+    a.skew = c->placement_skew;
     a.down = 0;
     a.iter = 1;
     a.px = patch_x(c);
@@ -5933,6 +5959,9 @@ extern "C" int fmm3d_set_option(fmm3d_ctx* c, const char* key, double v)
     } else if (!strcmp(key, "spin_limit")) {
         if (iv < 0 || iv > 10000000) return fail(c, FMM3D_E_ARG, "spin_limit out of range");
         c->spin_limit = iv;
+    } else if (!strcmp(key, "placement_skew")) {
+        if (iv < 0 || iv > 7) return fail(c, FMM3D_E_ARG, "placement_skew must be 0 .. 7");
+        c->placement_skew = iv;
     } else if (!strcmp(key, "autotune")) {
         if (iv != 0 && iv != 1) return fail(c, FMM3D_E_ARG, "autotune must be 0 or 1");
         c->autotune = iv;
