@@ -40,12 +40,17 @@ FMM3D_HD LookLate look_late(int ix, int iz, int snx, int snz, int px, int pz, in
     return r;
 }
 
-// The column a lane reads for itself (dx = dz = 0) or as a late input, counted
-// from two rows before the wavefront's first column (so that it is never
-// negative).  A lane without a column of its own reads the wavefront's first.
-FMM3D_HD unsigned look_node(int nnz, int lane, bool on, int dx, int dz)
+// Columns are counted from this many rows before the wavefront's first one: 2,
+// so that those of late inputs are not negative.  0 where a row is so long
+// that two of them on either side pass 32 bits of bytes: the check then reads
+// no late inputs and evaluates every node.
+FMM3D_HD int look_rows(int nnz, size_t bytes) { return ((size_t)4 * nnz + 64) * bytes <= 0xffffffffu ? 2 : 0; }
+
+// The column a lane reads for itself (dx = dz = 0) or as a late input (rows 2).
+// A lane without a column of its own reads the wavefront's first.
+FMM3D_HD unsigned look_node(int rows, int nnz, int lane, bool on, int dx, int dz)
 {
-    return on ? (unsigned)((2 + dx) * nnz + lane + dz) : 2u * (unsigned)nnz;
+    return on ? (unsigned)((rows + dx) * nnz + lane + dz) : (unsigned)(rows * nnz);
 }
 
 }  // namespace fmm3d

@@ -1570,6 +1570,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
     const R inf = Lim<R>::inf();
     const R hr = a.hr, ihr = R(1) / a.hr;
     const size_t nb = (NL + 255) / 256;   // blocks of columns per slot
+    const int rows = look_rows(a.nnz, sizeof(R));
     constexpr int B = 4;   // layers looked at together
     __shared__ unsigned queues[4][64 * B + 64];
     const int lane = threadIdx.x & 63;
@@ -1603,7 +1604,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         // the patch it waited for on that axis -- and only if that input is
         // not above it (the update counts no neighbour above its result).
         // Nodes with no such input are not evaluated.
-        const bool vf = a.vfilter && (a.born || iter == 1);
+        const bool vf = a.vfilter && rows && (a.born || iter == 1);
         const bool down = a.walkalt ? false : (a.down != 0);
         LookLate late = { { 0, 0 }, { 0, 0 } };
         if (vf && on) {
@@ -1628,14 +1629,14 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         unsigned ox[2], oz[2];
         R sx[2], sz[2];
         bool any_x[2], any_z[2];
-        const unsigned fo = look_node(a.nnz, lane, on, 0, 0);
+        const unsigned fo = look_node(rows, a.nnz, lane, on, 0, 0);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int dx = late.dx[k], dz = late.dz[k];
             any_x[k] = __ballot(dx != 0) != 0;
             any_z[k] = __ballot(dz != 0) != 0;
-            ox[k] = look_node(a.nnz, lane, on, dx, 0);
-            oz[k] = look_node(a.nnz, lane, on, 0, dz);
+            ox[k] = look_node(rows, a.nnz, lane, on, dx, 0);
+            oz[k] = look_node(rows, a.nnz, lane, on, 0, dz);
             sx[k] = dx ? (R)dx * rst.gx : inf;
             sz[k] = dz ? (R)dz * rst.gz : inf;
         }
@@ -1677,7 +1678,7 @@ __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
         // B layers at a time, their loads in flight together:
         // w[j] = layer ir - 2 + j of this column
         R w[B + 5];
-        const R* Tw = T + (ptrdiff_t)f0 - 2 * (ptrdiff_t)a.nnz;
+        const R* Tw = T + (ptrdiff_t)f0 - rows * (ptrdiff_t)a.nnz;
         auto at = [&](int ir, unsigned o) { return lane_load(Tw + (size_t)min(ir, snr - 1) * NL, o); };
         w[0] = inf; w[1] = inf;
         for (int j = 0; j < 3; ++j) w[2 + j] = j < snr ? at(j, fo) : inf;

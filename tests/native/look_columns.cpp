@@ -25,7 +25,7 @@ extern "C" void look_extent(int nnx, int nnz, int snx, int snz, int px, int pz, 
                 if (on) late = look_late(ix, iz, snx, snz, px, pz, fx, fz);
                 const long long base = (long long)f0 - 2 * (long long)nnz;
                 auto read = [&](int dx, int dz) {
-                    const long long c = base + look_node(nnz, lane, on, dx, dz);
+                    const long long c = base + look_node(2, nnz, lane, on, dx, dz);
                     lo = c < lo ? c : lo;
                     hi = c > hi ? c : hi;
                     return c;
@@ -42,4 +42,19 @@ extern "C" void look_extent(int nnx, int nnz, int snx, int snz, int px, int pz, 
     out[1] = hi;
     out[2] = own;
     out[3] = wrong;
+}
+
+// Whether every offset a lane of a wavefront forms for rows nnz long, times the
+// size of a value, is the exact one in 32 bits.
+extern "C" int look_fits(int nnz, int bytes)
+{
+    const int rows = look_rows(nnz, (size_t)bytes);
+    for (int lane = 0; lane < 64; ++lane)
+        for (int dx = -rows; dx <= rows; ++dx)
+            for (int dz = rows ? -2 : 0; dz <= (rows ? 2 : 0); ++dz) {
+                const unsigned o = look_node(rows, nnz, lane, true, dx, dz);
+                const long long exact = (long long)(rows + dx) * nnz + lane + dz;
+                if (exact >= 0 && (unsigned long long)(o * (unsigned)bytes) != (unsigned long long)exact * (unsigned)bytes) return 0;
+            }
+    return 1;
 }

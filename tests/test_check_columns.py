@@ -21,6 +21,7 @@ def extent(tmp_path_factory):
         out = (ctypes.c_longlong * 4)()
         so.look_extent(*args, out)
         return list(out)
+    call.fits = so.look_fits
     return call
 
 
@@ -41,3 +42,11 @@ def test_every_column_read_is_the_slots(extent, nnx, nnz):
                 lo, hi, own, wrong = extent(nnx, nnz, snx, snz, px, pz, fx, fz)
                 assert lo >= 0 and hi < nnx * nnz, (px, pz, fx, fz, snx, snz, lo, hi)
                 assert own == snx * snz and wrong == 0
+
+
+@pytest.mark.parametrize("nbytes", [4, 8])
+def test_offsets_of_long_rows_fit(extent, nbytes):
+    """An offset in 32 bits of bytes is the exact one whatever the rows' length."""
+    edge = ((1 << 32) - 1) // nbytes // 4 - 16   # the longest rows counted from two rows before
+    for nnz in (3, 140, 65536, edge - 1, edge, edge + 1, 1 << 27, 1 << 28, (1 << 29) + 5, (1 << 31) - 1):
+        assert extent.fits(nnz, nbytes), nnz
