@@ -275,6 +275,9 @@ int fmm3d_get_stats(const fmm3d_ctx *ctx, fmm3d_stats *out);
  *                   four times as many where the neighbour's progress is
  *                   in the same XCD's cache); also of the waits between
  *                   patches in the reference-partition mode
+ *   "one_node"      column walk on 8x8 patches: 1 (default) one node per lane;
+ *                   0 the walk of the other patches, which layers of 2^32
+ *                   bytes and more take in any case (same fields, slower)
  *   "placement_skew" column walk: XCDs between consecutive patches of a
  *                   source whose first sweep is meant for one XCD (0..7,
  *                   default 0); other values show that a placement that

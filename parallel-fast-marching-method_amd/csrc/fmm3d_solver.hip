@@ -2464,6 +2464,7 @@ struct fmm3d_ctx {
     std::vector<float> eng_hout;
     int ordered = 1;               // column walk: patches wait for their upstream neighbours
     int spin_limit = 20000;        // polls (~64 cycles each) before such a wait is given up
+    int one_node = 1;              // 8 x 8 patches: one node per lane (k_walk8), where its offsets reach
     int placement_skew = 0;        // XCDs between consecutive patches of a slot meant to lie on one (tests)
     int max_sweeps = 0;            // column walk: stop after this many sweeps (0: at convergence)
     bool walk_settled = true;      // the last column-walk solve ended at its fixed point (not at max_sweeps)
@@ -3415,10 +3416,12 @@ static int sweep_kernel(const fmm3d_ctx* c, int k, bool engine)
 }
 
 // Whether k_walk8 walks the columns: one node per lane, and 32-bit byte
-// offsets within a layer.
-template <typename R> static bool column_one_node(const ColArgs<R>& a)
+// offsets within a layer.  Larger layers take k_column's 8 x 8 form, whose
+// addresses are 64-bit ones (a float64 source at 201^3: 4.0 ms against 3.35; 50
+// float32 ones: 22.5 against 15.3).
+template <typename R> static bool column_one_node(const fmm3d_ctx* c, const ColArgs<R>& a)
 {
-    return a.px == 8 && a.pz == 8 && (size_t)a.nnx * a.nnz * sizeof(R) <= 0xffffffffu;
+    return c->one_node && a.px == 8 && a.pz == 8 && (size_t)a.nnx * a.nnz * sizeof(R) <= 0xffffffffu;
 }
 
 template <typename R, bool FAST, bool SHIFT>
@@ -3433,7 +3436,7 @@ static hipError_t launch_column(fmm3d_ctx* c, const ColArgs<R>& a, int blocks, i
         return hipGetLastError();
     }
     const int px = patch_x(c), pz = patch_z(c);   // the hyperplane strategy's patches are 8 x 8
-    if (column_one_node(a)) {
+    if (column_one_node(c, a)) {
         k_walk8<R, FAST, SHIFT><<<blocks, 64, 0, c->stream>>>(a);
         return hipGetLastError();
     }
@@ -3612,13 +3615,13 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
     }
     a.iter = 0;
     a.iterp = c->d_iter;
-    std::vector<char> sig(sizeof a + 4 * sizeof(int));
+    std::vector<char> sig(sizeof a + 5 * sizeof(int));
     memcpy(sig.data(), &a, sizeof a);
     // the walk mode decides whether the graph holds the fixed-point check;
     // n is the sweeps the graph holds (a graph of fewer sweeps replayed for
     // a longer chunk would skip sweeps)
-    const int tag[4] = { blocks, (int)sizeof(R) * 100 + kind * 10000000 + c->strategy * 1000000 +
-                                     c->plane_ch * 100000 + c->col_px * 10000 + c->col_pz, c->walk_alt, n };
+    const int tag[5] = { blocks, (int)sizeof(R) * 100 + kind * 10000000 + c->strategy * 1000000 +
+                                     c->plane_ch * 100000 + c->col_px * 10000 + c->col_pz, c->walk_alt, n, c->one_node };
     memcpy(sig.data() + sizeof a, tag, sizeof tag);
     if (!c->gexec || sig != c->g_sig) {
         if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
@@ -4649,6 +4652,7 @@ static int point_group(const fmm3d_ctx* c, fmm3d_ctx** finep, std::string& err, 
     }
     fc->g = cg;
     fc->point_order = c->point_order;
+    fc->one_node = c->one_node;
     fc->point_window = c->point_window;
     // the vertex model (its gridding onto the shared arrays goes unused:
     // every slot has its own block)
@@ -5737,6 +5741,9 @@ extern "C" int fmm3d_set_option(fmm3d_ctx* c, const char* key, double v)
     } else if (!strcmp(key, "spin_limit")) {
         if (iv < 0 || iv > 10000000) return fail(c, FMM3D_E_ARG, "spin_limit out of range");
         c->spin_limit = iv;
+    } else if (!strcmp(key, "one_node")) {
+        if (iv != 0 && iv != 1) return fail(c, FMM3D_E_ARG, "one_node must be 0 or 1");
+        c->one_node = iv;
     } else if (!strcmp(key, "placement_skew")) {
         if (iv < 0 || iv > 7) return fail(c, FMM3D_E_ARG, "placement_skew must be 0 .. 7");
         c->placement_skew = iv;
