@@ -86,16 +86,47 @@ template <int J> __device__ __forceinline__ float add16(float s, float p)
     return s + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p), 0x150 + J, 0xf, 0xf, false));   // row_newbcast:J
 }
 
+// The sum of one list's products, its entries k .. k1 - 1 in order: every lane
+// of the 16 that share the list gets it (l: the lane's place in them).  They
+// load and multiply 64 entries side by side, and each then adds the 64 products
+// in order, so only the additions are serial, one instruction for an entry of
+// each of the wavefront's four lists.  (An entry past the end adds +0, which
+// changes no sum: one that starts from +0 is never -0.)
+__device__ __forceinline__ float list_sum16(int64_t k, int64_t k1, int l, const int32_t* __restrict__ idx,
+                                            const float* __restrict__ val, const float* __restrict__ x)
+{
+    float s = 0.0f;
+    int32_t c[4];
+    float v[4];
+    auto fetch = [&](int64_t at) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t e = at + 16 * j + l;
+            const bool in = e < k1;
+            c[j] = in ? idx[e] : -1;
+            v[j] = in ? val[e] : 0.0f;
+        }
+    };
+    fetch(k);
+    while (__ballot(k < k1)) {
+        float p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = c[j] >= 0 ? v[j] * x[c[j]] : 0.0f;
+        k += 64;
+        fetch(k);   // the next entries are on their way during the sum
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s = add16<15>(s, p[j]);
+    }
+    return s;
+}
+
 // y(i) = (sum over list i of val(k) x(idx(k)), in list order) / cd(i): G^T x over
 // the columns, rows ascending (subinv.f90:612-616), G x / cd over the rows, in
-// file order (subinv.f90:759-767).  Sixteen lanes per list: they load and
-// multiply 64 entries side by side, and each then adds the 64 products in
-// order, so only the additions are serial, one instruction for an entry of each
-// of the wavefront's four lists.  (An entry past the end adds +0, which changes
-// no sum: one that starts from +0 is never -0.)  Bound by latency: a list of
-// 250 entries is four rounds of two dependent loads.  15000 x 19683, 3.75M
-// entries, G^T x and G x: one thread per list, its loads a list apart, 594 and
-// 151 us; one wavefront per list, two instructions an entry, 45 each; 23 so.
+// file order (subinv.f90:759-767).  Sixteen lanes per list.  Bound by latency:
+// a list of 250 entries is four rounds of two dependent loads.  15000 x 19683,
+// 3.75M entries, G^T x and G x: one thread per list, its loads a list apart,
+// 594 and 151 us; one wavefront per list, two instructions an entry, 45 each;
+// 23 so.
 __global__ void __launch_bounds__(256) k_ordered_sums(int64_t n, const int64_t* __restrict__ ptr, const int32_t* __restrict__ idx,
                                                       const float* __restrict__ val, const float* __restrict__ x,
                                                       const float* __restrict__ cd, float* __restrict__ y)
@@ -107,34 +138,60 @@ __global__ void __launch_bounds__(256) k_ordered_sums(int64_t n, const int64_t* 
         const int64_t i = i0 + ((threadIdx.x >> 4) & 3);
         int64_t k = 0, k1 = 0;
         if (i < n) { k = ptr[i]; k1 = ptr[i + 1]; }
-        float s = 0.0f;
-        int32_t c[4];
-        float v[4];
-        auto fetch = [&](int64_t at) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t e = at + 16 * j + l;
-                const bool in = e < k1;
-                c[j] = in ? idx[e] : -1;
-                v[j] = in ? val[e] : 0.0f;
-            }
-        };
-        fetch(k);
-        while (__ballot(k < k1)) {
-            float p[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) p[j] = c[j] >= 0 ? v[j] * x[c[j]] : 0.0f;
-            k += 64;
-            fetch(k);   // the next entries are on their way during the sum
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s = add16<15>(s, p[j]);
-        }
+        const float s = list_sum16(k, k1, l, idx, val, x);
         if (l == 0 && i < n) y[i] = cd ? s / cd[i] : s;
     }
 }
 
+// The same where lists are short on average: a lane per list of at most
+// SHORT_LIST entries, then the wavefront's longer ones, four at a time.
+constexpr int SHORT_LIST = 32;
+__global__ void __launch_bounds__(256) k_ordered_sums_short(int64_t n, const int64_t* __restrict__ ptr, const int32_t* __restrict__ idx,
+                                                            const float* __restrict__ val, const float* __restrict__ x,
+                                                            const float* __restrict__ cd, float* __restrict__ y)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t step = (int64_t)gridDim.x * 256;
+    for (int64_t i0 = blockIdx.x * (int64_t)256 + (threadIdx.x & ~63); i0 < n; i0 += step) {
+        const int64_t i = i0 + lane;
+        int64_t k = 0, k1 = 0;
+        if (i < n) { k = ptr[i]; k1 = ptr[i + 1]; }
+        const bool small = k1 - k <= SHORT_LIST;
+        if (i < n && small) {
+            float s = 0.0f;
+            for (int64_t e = k; e < k1; ++e) s = s + val[e] * x[idx[e]];
+            y[i] = cd ? s / cd[i] : s;
+        }
+        for (unsigned long long left = __ballot(!small); left;) {
+            // the 16 lanes' list: of those left, as many taken before as lower sixteens
+            unsigned long long own = left;
+            for (int g = 0; g < 4; ++g) {
+                if (g < lane >> 4) own &= own - 1;
+                left &= left - 1;
+            }
+            const int from = own ? __ffsll(own) - 1 : 0;
+            const int64_t a = __shfl(k, from), b = __shfl(k1, from);
+            const float s = list_sum16(a, own ? b : a, lane & 15, idx, val, x);
+            if (own && (lane & 15) == 0) y[i0 + from] = cd ? s / cd[i0 + from] : s;
+        }
+    }
+}
+
 int grid_of(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 65536); }
-int lists_grid(int64_t n) { return (int)std::min<int64_t>((n + 15) / 16, 65536); }
+
+// Lists of fewer than this many entries on average take a lane each.  A call
+// with sixteen lanes a list / a lane a list, us: 1,000,000 rows of 2 entries
+// 479 / 406, of 4 471 / 437, of 8 479 / 451, 500,000 of 16 254 / 315; the
+// columns of 1,000,000, mean 0.1 (few rows of a large model) 322 / 289, 2
+// 352 / 311, 8 348 / 346, 16 385 / 517.
+constexpr int SHORT_MEAN = 8;
+
+void ordered_sums(hipStream_t st, int64_t n, int64_t nnz, const int64_t* ptr, const int32_t* idx, const float* val,
+                  const float* x, const float* cd, float* y)
+{
+    if (nnz < SHORT_MEAN * n) k_ordered_sums_short<<<grid_of(n), 256, 0, st>>>(n, ptr, idx, val, x, cd, y);
+    else k_ordered_sums<<<(int)std::min<int64_t>((n + 15) / 16, 65536), 256, 0, st>>>(n, ptr, idx, val, x, cd, y);
+}
 
 }  // namespace
 
@@ -241,7 +298,7 @@ extern "C" int fmm3d_gmat_gtx(fmm3d_gmat* m, const float* x, float* y)
     hipError_t e = hipSetDevice(m->device);
     if (e == hipSuccess && m->nrows) e = hipMemcpyAsync(m->x, x, m->nrows * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess) {
-        k_ordered_sums<<<lists_grid(m->ncols), 256, 0, m->stream>>>(m->ncols, m->cp, m->row, m->tval, m->x, nullptr, m->y);
+        ordered_sums(m->stream, m->ncols, m->nnz, m->cp, m->row, m->tval, m->x, nullptr, m->y);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(y, m->y, m->ncols * sizeof(float), hipMemcpyDeviceToHost, m->stream);
@@ -257,7 +314,7 @@ extern "C" int fmm3d_gmat_gx(fmm3d_gmat* m, const float* x, const float* cd, flo
     if (e == hipSuccess) e = hipMemcpyAsync(m->x, x, m->ncols * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess && cd && m->nrows) e = hipMemcpyAsync(m->cd, cd, m->nrows * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess && m->nrows) {
-        k_ordered_sums<<<lists_grid(m->nrows), 256, 0, m->stream>>>(m->nrows, m->rp, m->col, m->val, m->x, cd ? m->cd : nullptr, m->y);
+        ordered_sums(m->stream, m->nrows, m->nnz, m->rp, m->col, m->val, m->x, cd ? m->cd : nullptr, m->y);
         e = hipGetLastError();
     }
     if (e == hipSuccess && m->nrows) e = hipMemcpyAsync(y, m->y, m->nrows * sizeof(float), hipMemcpyDeviceToHost, m->stream);
