@@ -957,7 +957,7 @@ k_column(ColArgs<R> a)
                     };
                     const R h[3] = { hr, hxl, shz[lx] };
                     const R ih[3] = { ihr, ihx, sihz[lx] };
-                    const R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown), rq);
+                    const R nv = ref_round(col_update<R, FAST, SHIFT, FAST>(a.fom, tc, gather, h, ih, slown), rq);
                     // every lane has read its stencil before any lane writes (one wavefront)
                     __builtin_amdgcn_wave_barrier();
                     if (nv != tc) {
@@ -1238,7 +1238,13 @@ k_walk8(ColArgs<R> a)
             cur[ridx] = hv;
             __builtin_amdgcn_wave_barrier();
             // passes until one changes nothing (slots with a reference: moves
-            // no node by more than ptl), as k_column's
+            // no node by more than ptl), as k_column's.  In float32, once a
+            // pass needs more than one octant for some node, the layer's later
+            // ones take all eight at once: they mostly need them too, and a
+            // chain of one octant and then others is longer than eight side by
+            // side (61x300x61, 4 sources: 3.71 ms without this, 2.54 with;
+            // 300x61x61, 3: 11.2, 7.4; 201^3, 50: 14.0, 13.4).
+            bool eight = false;
             int npass = 0;
 #pragma unroll 1
             for (int pass = 0; pass < a.maxpass; ++pass) {
@@ -1256,8 +1262,14 @@ k_walk8(ColArgs<R> a)
                     }
                     return g;
                 };
-                R nv = ref_round(col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown, free), rq);
-                nv = free ? nv : tc;
+                R nv;
+                if constexpr (FAST) {
+                    if (eight) nv = col_update<R, FAST, SHIFT, true>(a.fom, tc, gather, h, ih, slown, free);
+                    else nv = col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown, free, &eight);
+                } else {
+                    nv = col_update<R, FAST, SHIFT>(a.fom, tc, gather, h, ih, slown, free);
+                }
+                nv = free ? ref_round(nv, rq) : tc;
                 // every lane has read its stencil before any lane writes (one wavefront)
                 __builtin_amdgcn_wave_barrier();
                 const bool moved = nv != tc && !(fabs(nv - tc) <= ptl);
@@ -1777,7 +1789,7 @@ k_plane(ColArgs<R> a)
                     };
                     const R h[3] = { hr, qhx[q], qhz[q] };
                     const R ih[3] = { ihr, fast_rcp(qhx[q]), fast_rcp(qhz[q]) };
-                    const R nv = col_update<R, FAST, SHIFT>(a.fom, C0, gather, h, ih, qs[q]);
+                    const R nv = col_update<R, FAST, SHIFT, FAST>(a.fom, C0, gather, h, ih, qs[q]);
                     ++nupd;
                     if (nv != C0) {
                         cur = nv;

@@ -90,6 +90,46 @@ __device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], cons
     }
 }
 
+// All eight octants in the axis-sum form, side by side: cheap in float32 (a
+// hardware square root and reciprocal each).  Per side (a, b, c) = (alpha^2,
+// alpha*beta, beta^2); a missing side carries a = NaN, and fmin passes over the
+// octants through it.
+template <typename R, bool SHIFT, typename G>
+__device__ __forceinline__ R octants_eight(int fom, R top, R sh, G gather, const R ih[3], R s2)
+{
+    struct Coef { R a, b, c; };
+    auto coef = [&](R w1, R w2, bool in, R ihx) {
+        // selects on plain values keep this branch-free
+        const bool cnt = SHIFT ? w1 <= top : w1 < top, sec = fom && w1 > w2;
+        const R u1 = w1 - sh, u2 = w2 - sh;
+        const R num = sec ? fma(R(-0.5), u2, u1 + u1) : u1;
+        const R al = ihx * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
+        const R be = cnt ? num * ihx : R(0);
+        return Coef{ in ? al * al : R(__builtin_nan("")), al * be, be * be };
+    };
+    R best = Lim<R>::inf();
+    const AxisSides<R> r = gather(0), x = gather(1), z = gather(2);
+    Coef cr[2] = { coef(r.l1, r.l2, r.lin, ih[0]), coef(r.h1, r.h2, r.hin, ih[0]) };
+    const Coef cx[2] = { coef(x.l1, x.l2, x.lin, ih[1]), coef(x.h1, x.h2, x.hin, ih[1]) };
+    const Coef cz[2] = { coef(z.l1, z.l2, z.lin, ih[2]), coef(z.h1, z.h2, z.hin, ih[2]) };
+    cr[0].c -= s2;
+    cr[1].c -= s2;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const R Axz = cx[j].a + cz[k].a, Bxz = cx[j].b + cz[k].b, Cxz = cx[j].c + cz[k].c;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const R A = cr[i].a + Axz, B = cr[i].b + Bxz, C = cr[i].c + Cxz;
+                R disc = fused_mul_sub(B, B, A * C);
+                disc = disc > R(0) ? disc : R(0);
+                best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
+            }
+        }
+    return best;
+}
+
 // The minimum over the octants of a node whose one octant, of solution best,
 // was not certain on the axes weak, or has both sides of an axis counted
 // (sides counted below top, times relative to sh).  Per axis, role 0 is the
@@ -122,39 +162,7 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
     unsigned unsure = weak & drop;
     if constexpr (FAST) {
         if (__any(__popc(both | unsure) > 1)) {
-            // an octant is cheap here (a hardware square root and reciprocal):
-            // all eight, one theta side and one phi side at a time.  Per side
-            // (a, b, c) = (alpha^2, alpha*beta, beta^2); a missing side carries
-            // a = NaN, and fmin passes over the octants through it
-            struct Coef { R a, b, c; };
-            auto coef = [&](R w1, R w2, bool in, R ihx) {
-                // selects on plain values keep this branch-free
-                const bool cnt = counts(w1), sec = fom && w1 > w2;
-                const R u1 = w1 - sh, u2 = w2 - sh;
-                const R num = sec ? fma(R(-0.5), u2, u1 + u1) : u1;
-                const R al = ihx * (cnt ? (sec ? R(1.5) : R(1)) : R(0));
-                const R be = cnt ? num * ihx : R(0);
-                return Coef{ in ? al * al : R(__builtin_nan("")), al * be, be * be };
-            };
-#pragma unroll 1
-            for (int o = 0; o < 4; ++o) {
-                asm volatile("" ::: "memory");   // the stencil is read again, not kept
-                const AxisSides<R> r = gather(0), x = gather(1), z = gather(2);
-                const bool hx = o & 1, hz = o & 2;
-                const Coef cx = coef(hx ? x.h1 : x.l1, hx ? x.h2 : x.l2, hx ? x.hin : x.lin, ih[1]);
-                const Coef cz = coef(hz ? z.h1 : z.l1, hz ? z.h2 : z.l2, hz ? z.hin : z.lin, ih[2]);
-                const Coef c0 = coef(r.l1, r.l2, r.lin, ih[0]), c1 = coef(r.h1, r.h2, r.hin, ih[0]);
-                const R Axz = cx.a + cz.a, Bxz = cx.b + cz.b, Cxz = cx.c + cz.c;
-                auto octant = [&](const Coef& c) {
-                    const R A = c.a + Axz, B = c.b + Bxz, C = (c.c - s2) + Cxz;
-                    R disc = fused_mul_sub(B, B, A * C);
-                    disc = disc > R(0) ? disc : R(0);
-                    best = fmin(best, (B + fast_sqrt(disc)) * fast_rcp(A));
-                };
-                octant(c0);
-                octant(c1);
-            }
-            return best;
+            return octants_eight<R, SHIFT>(fom, top, sh, gather, ih, s2);
         }
     }
     best = one;
@@ -191,8 +199,15 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
 // the reference's leading-axis form in the CPU oracle's operation order.
 // h, ih: spacings and their reciprocals along r, x, z.  free: whether the node
 // is one to update (the value returned for another one is not to be used).
-template <typename R, bool FAST, bool SHIFT, typename G>
-__device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], const R ih[3], R slown, bool free = true)
+// EIGHT (float32): all eight octants at once.  *more, if asked for: whether one
+// octant left some node of the wavefront in doubt.
+// The walks whose lanes hold more than one node, and the hyperplane walk, take
+// eight in float32: their many nodes a wavefront leave few passes where one
+// decides (201^3, 20 sources, 16 x 16 patches / 8 x 16 / hyperplane, a call:
+// 19.0 / 13.4 / 122 ms with one octant first, 15.8 / 12.1 / 90.6 so).
+template <typename R, bool FAST, bool SHIFT, bool EIGHT = false, typename G>
+__device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], const R ih[3], R slown, bool free = true,
+                                        bool* more = nullptr)
 {
     const R inf = Lim<R>::inf();
     // per axis the lower side (t1, t2) -- the counted one, where one counts --
@@ -225,9 +240,16 @@ __device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], c
         p[a].t2 = FAST || p[a].ord == 2 ? t2[a] - sh : R(0);
         kt += R(0x1.2p-38) * ih[a] * ih[a];   // the largest (c / H)^2: 9/4
     }
-    unsigned weak;
-    R best = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
-    if ((weak || counts(other)) && known && free) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt, best, weak);
+    R best;
+    if constexpr (EIGHT) {
+        best = octants_eight<R, SHIFT>(fom, top, sh, gather, ih, s2);
+    } else {
+        unsigned weak;
+        best = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
+        const bool doubt = (weak || counts(other)) && known && free;
+        if (more) *more = __any(doubt);
+        if (doubt) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt, best, weak);
+    }
     if (SHIFT && best < inf) best = sh + best;
     return known ? best : inf;
 }

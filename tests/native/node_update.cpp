@@ -130,7 +130,8 @@ void run(long n, unsigned seed, int fom, long long* out)
         bool clamped = false;
         const R want = eight<R, FAST, SHIFT>(fom, d, &nlow, &clamped);
         const R got = col_update<R, FAST, SHIFT>(fom, d.tc, gather, d.h, ih, d.slown);
-        out[0] += !same(want, got);
+        const R all = col_update<R, FAST, SHIFT, FAST>(fom, d.tc, gather, d.h, ih, d.slown);
+        out[0] += !same(want, got) || !same(want, all);
         for (int a = 0; a < 3; ++a) {
             two |= d.v1[a][0] < d.tc && d.v1[a][1] < d.tc;
             outside |= !d.in[a][0] || !d.in[a][1];
