@@ -1651,17 +1651,15 @@ k_plane(ColArgs<R> a)
     const size_t col = mine ? (size_t)gx * a.nnz + gz : 0;
     const int hzrow = min(gx, a.nnx - 1);
     // Per-lane flags, packed in one register and rebuilt at each use (as
-    // lane masks they would hold sixteen scalar register pairs through the
-    // step loop): bits 0-7 which lateral stencil sides exist (flow-upstream
-    // and downstream theta and phi, one and two nodes away), bits 8-15 which
-    // lateral neighbours come from the halo ring, bit 16 the column is in
-    // the grid.
+    // lane masks they would hold a scalar register pair each through the
+    // step loop): bits 0-3 which lateral neighbours exist (flow-upstream and
+    // downstream theta, then phi), bits 8-15 which lateral neighbours (one and
+    // two nodes away) come from the halo ring, bit 16 the column is in the
+    // grid.
     auto inr = [](int v, int n) { return v >= 0 && v < n; };
     const unsigned lane_flags =
-        (inr(gx - fx, a.nnx) ? 1u : 0u) | (inr(gx - 2 * fx, a.nnx) ? 2u : 0u) |
-        (inr(gx + fx, a.nnx) ? 4u : 0u) | (inr(gx + 2 * fx, a.nnx) ? 8u : 0u) |
-        (inr(gz - fz, a.nnz) ? 16u : 0u) | (inr(gz - 2 * fz, a.nnz) ? 32u : 0u) |
-        (inr(gz + fz, a.nnz) ? 64u : 0u) | (inr(gz + 2 * fz, a.nnz) ? 128u : 0u) |
+        (inr(gx - fx, a.nnx) ? 1u : 0u) | (inr(gx + fx, a.nnx) ? 2u : 0u) |
+        (inr(gz - fz, a.nnz) ? 4u : 0u) | (inr(gz + fz, a.nnz) ? 8u : 0u) |
         (li == 0 ? 0x100u : 0u) | (li <= 1 ? 0x200u : 0u) | (li == P - 1 ? 0x400u : 0u) | (li >= P - 2 ? 0x800u : 0u) |
         (lj == 0 ? 0x1000u : 0u) | (lj <= 1 ? 0x2000u : 0u) | (lj == P - 1 ? 0x4000u : 0u) | (lj >= P - 2 ? 0x8000u : 0u) |
         (gx < a.nnx && gz < a.nnz ? 0x10000u : 0u);
@@ -1783,8 +1781,8 @@ k_plane(ColArgs<R> a)
                     auto gather = [&](int ax) {
                         AxisSides<R> g;
                         if (ax == 0) g = { down ? P1 : N1, down ? P2 : N2, down ? N1 : P1, down ? N2 : P2, ir >= 1, ir + 1 < nr };
-                        else if (ax == 1) g = { xm1, xm2, xp1, xp2, (lf & 1u) != 0, (lf & 4u) != 0 };
-                        else g = { zm1, zm2, zp1, zp2, (lf & 16u) != 0, (lf & 64u) != 0 };
+                        else if (ax == 1) g = { xm1, xm2, xp1, xp2, (lf & 1u) != 0, (lf & 2u) != 0 };
+                        else g = { zm1, zm2, zp1, zp2, (lf & 4u) != 0, (lf & 8u) != 0 };
                         return g;
                     };
                     const R h[3] = { hr, qhx[q], qhz[q] };
