@@ -409,7 +409,7 @@ template <typename R> struct ColArgs {
     int nnr, nnx, nnz;
     int npx, npz;           // patches per axis
     int nslots;
-    const int* act;         // 8 x 8 patches: the slots of this sweep (k_next_sweep)
+    int* act;               // 8 x 8 patches: the slots of this sweep (k_next_sweep), or null: all, spread
     int iter;
     int fom;
     int maxpass;            // line passes per layer at most (cycle +phi, -phi, +theta, -theta)
@@ -1071,7 +1071,7 @@ k_walk8(ColArgs<R> a)
     // store visible, and the fixed-point check then trusts no neighbour of the
     // slot to have been waited for.
     const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int nspread = uniform_load(a.act, 0), nlocal = uniform_load(a.act, 1);
+    const int nspread = a.act ? uniform_load(a.act, 0) : a.nslots, nlocal = a.act ? uniform_load(a.act, 1) : 0;
     const int kspread = (nspread * a.npx + 7) / 8 * a.npz;
     const bool local = k >= kspread;
     int slot, rank;   // the patch's launch rank in its slot
@@ -1086,7 +1086,7 @@ k_walk8(ColArgs<R> a)
         slot = row / a.npx;
         rank = row % a.npx * a.npz + k % a.npz;
     }
-    slot = uniform_load(a.act, 2 + slot);
+    if (a.act) slot = uniform_load(a.act, 2 + slot);
     if (!a.slot_on[slot]) return;
     const int iter = a.iterp ? __hip_atomic_load(a.iterp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.iter;
     int bx, bz, fx, fz;
@@ -3592,7 +3592,12 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         for (int j = 0; j < n; ++j) {
             a.iter = k + j;
             const int kd = sweep_kernel(c, k + j, engine);
-            k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
+            // fewer than eight slots are spread in any case: their patches
+            // return by themselves where nothing changed, without a launch
+            // before each sweep that lists the slots
+            a.act = kd == 1 && a.nslots >= 8 && column_one_node(c, a) ? c->sl.act : nullptr;
+            if (a.act)
+                k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, a.act);
             if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j], c->stream));
             hipError_t le = launch_column<R, FAST, SHIFT>(c, a, blocks, kd);
             HIPCHK(c, le);
