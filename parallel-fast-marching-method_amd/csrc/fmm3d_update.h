@@ -46,8 +46,8 @@ template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return _
 // M = A T^2 + sum beta^2 + s^2 <= 3 (sum beta^2 + s^2); the margin asked for
 // is 2^8 of them.  Where an axis' term is not certain, the octant without it
 // is evaluated too, and where both sides of an axis count, the octants of
-// either, so that every value is the minimum over all eight octants to the
-// last bit.  Measured against eight octants each time: 6 % of the wavefronts'
+// either (float32: all eight in either case), so that every value is the
+// minimum over all eight octants to the last bit.  Measured against eight octants each time: 6 % of the wavefronts'
 // passes need more than one in the first sweep of 50 float32 plane waves at
 // 201^3, which went from 5.55 to 3.53 G VALU instructions; in k_column, eight
 // float64 sources at 31x110x140 went from 9.0 to 5.4 ms and a local source at
@@ -91,7 +91,9 @@ __device__ __forceinline__ R octant_eval(const Side<R> p[3], const R h2[3], cons
 }
 
 // All eight octants in the axis-sum form, side by side: cheap in float32 (a
-// hardware square root and reciprocal each).  Per side (a, b, c) = (alpha^2,
+// hardware square root and reciprocal each), where a node's own, one after the
+// other, gained nothing (201^3, 50 plane waves, a solve: 13.4 ms with those
+// where one axis is in doubt, 13.2 so).  Per side (a, b, c) = (alpha^2,
 // alpha*beta, beta^2); a missing side carries a = NaN, and fmin passes over the
 // octants through it.
 template <typename R, bool SHIFT, typename G>
@@ -132,25 +134,22 @@ __device__ __forceinline__ R octants_eight(int fom, R top, R sh, G gather, const
 
 // The minimum over the octants of a node whose one octant, of solution best,
 // was not certain on the axes weak, or has both sides of an axis counted
-// (sides counted below top, times relative to sh).  Per axis, role 0 is the
-// lower side and role 1 the other: its octants differ where both sides count
-// (both), and where role 1 leaves the axis out while role 0 counts (drop).
-// The other octants of the counted sides come first, then those without one or
-// more of the axes some of them left uncertain; each lane goes through its own
-// (their sets differ from node to node), so the wavefront takes the most that
-// one node needs (float64, eight plane waves at 31x110x140, a call: 8.1 ms with
-// the set its nodes need together, 4.5 so; the first sweep took 5.2 ms with all
-// eight octants and 3.3 with that set).  Where a node of the wavefront has more
-// than one such axis, float32 takes all eight: they are cheap there side by side
-// (201^3, 50 plane waves / a refined source at 61^3, a call: 21.7 / 26.8 ms with
-// all eight always, 18.7 / 32.5 never, 18.6 / 25.9 so).  The stencil is gathered
-// again for each, so that this path holds few registers.
-template <typename R, bool FAST, bool SHIFT, typename G>
+// (sides counted below top, times relative to sh), where an octant is dear
+// (float64).  Per axis, role 0 is the lower side and role 1 the other: its
+// octants differ where both sides count (both), and where role 1 leaves the
+// axis out while role 0 counts (drop).  The other octants of the counted sides
+// come first, then those without one or more of the axes some of them left
+// uncertain; each lane goes through its own (their sets differ from node to
+// node), so the wavefront takes the most that one node needs (eight plane waves
+// at 31x110x140, a call: 8.1 ms with the set its nodes need together, 4.5 so;
+// the first sweep took 5.2 ms with all eight octants and 3.3 with that set).
+// The stencil is gathered again for each, so that this path holds few
+// registers.
+template <typename R, bool SHIFT, typename G>
 __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const R h2[3], const R ih[3], R s2, R kt,
-                                          R one, unsigned weak)
+                                          R best, unsigned weak)
 {
     auto counts = [&](R v) { return SHIFT ? v <= top : v < top; };
-    R best = Lim<R>::inf();
     unsigned both = 0, drop = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -160,12 +159,6 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
         drop |= !ob && counts(lo ? g.l1 : g.h1) && (lo ? g.hin : g.lin) ? 1u << a : 0u;
     }
     unsigned unsure = weak & drop;
-    if constexpr (FAST) {
-        if (__any(__popc(both | unsure) > 1)) {
-            return octants_eight<R, SHIFT>(fom, top, sh, gather, ih, s2);
-        }
-    }
-    best = one;
     // todo: the octants left, a bit for each set of axes in role 1
     unsigned todo = subsets(both) & ~1u;
     for (bool first = true;;) {
@@ -187,7 +180,7 @@ __device__ __forceinline__ R octants_more(int fom, R top, R sh, G gather, const 
         }
         if (!(p[0].ord | p[1].ord | p[2].ord)) continue;
         unsigned w;
-        const R T = octant_eval<R, FAST>(p, h2, ih, s2, kt, &w);
+        const R T = octant_eval<R, false>(p, h2, ih, s2, kt, &w);
         if (T < best) best = T;
         if (first) unsure |= w & drop;
     }
@@ -248,7 +241,10 @@ __device__ __forceinline__ R col_update(int fom, R tc, G gather, const R h[3], c
         best = octant_eval<R, FAST>(p, h2, ih, s2, kt, &weak);
         const bool doubt = (weak || counts(other)) && known && free;
         if (more) *more = __any(doubt);
-        if (doubt) best = octants_more<R, FAST, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt, best, weak);
+        if (doubt) {
+            if constexpr (FAST) best = octants_eight<R, SHIFT>(fom, top, sh, gather, ih, s2);
+            else best = octants_more<R, SHIFT>(fom, top, sh, gather, h2, ih, s2, kt, best, weak);
+        }
     }
     if (SHIFT && best < inf) best = sh + best;
     return known ? best : inf;

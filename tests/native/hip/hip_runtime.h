@@ -18,9 +18,7 @@ using std::sqrt;
 inline int __ffs(unsigned x) { return __builtin_ffs((int)x); }
 inline int __popc(unsigned x) { return __builtin_popcount(x); }
 
-// the wavefront's other lanes: whether one of them says yes
-extern bool lane_others;
-inline bool __any(bool x) { return x || lane_others; }
+inline bool __any(bool x) { return x; }
 
 // the hardware's square root and reciprocal are good to one unit in the last
 // place: lane_ulp moves a result by -1, 0 or 1 of them, by its argument's bits

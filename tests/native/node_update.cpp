@@ -8,7 +8,6 @@
 
 using namespace fmm3d;
 
-bool lane_others = false;
 int lane_ulp = 0;
 
 namespace {
@@ -146,9 +145,8 @@ void run(long n, unsigned seed, int fom, long long* out)
 
 }  // namespace
 
-extern "C" void node_update(int f32, int order, long n, unsigned seed, int others, int ulp, long long* out)
+extern "C" void node_update(int f32, int order, long n, unsigned seed, int ulp, long long* out)
 {
-    lane_others = others != 0;
     lane_ulp = ulp;
     for (int k = 0; k < 6; ++k) out[k] = 0;
     if (f32) run<float, true, true>(n, seed, order, out);
