@@ -47,7 +47,11 @@ extern "C" {
 #define FMM3D_ORDER_FIRST   0   /* first-order stencils (.in line 9 = 0)    */
 #define FMM3D_ORDER_MIXED   1   /* mixed first/second order (.in line 9 = 1) */
 #define FMM3D_PREC_FP64     0   /* float64 node updates                     */
-#define FMM3D_PREC_FP32     1   /* float32 updates on times offset by the source's boundary minimum */
+#define FMM3D_PREC_FP32     1   /* float32 updates on times offset by the source's boundary minimum.
+                                   * About one local source in a thousand, and plane waves in grids
+                                   * much finer laterally than in depth, never settle in float32: the
+                                   * solve returns FMM3D_E_NOCONV at its sweep cap, for the whole
+                                   * batch and without fields.  They settle in float64. */
 #define FMM3D_WALK_ALTERNATE 1  /* flag: column walk alternates bottom-up / top-down (point sources) */
 #define FMM3D_REFERENCE_PARTITION 2  /* fmm3d_solve_tele flag: the reference's 2x2x2 partitioned solve */
 

@@ -1040,12 +1040,13 @@ k_column(ColArgs<R> a)
 // on four sides, one per lane; no corners: the stencil is a cross) are waited
 // for when a layer is staged.  Halo cells outside the grid hold inf from the
 // start and are never written (their lanes write the spare cells behind).
-// Same passes, same order, same values as k_column.  A layer costs 400 VALU
-// instructions in float32 (565 in k_column<8, 8>, whose per-lane 64-bit
-// addresses, lane masks and LDS window it does without) and 15 passes of 225
-// each in float64, where the 8 + 8 nodes of a patch's longest chain set the
-// time: 1.45 k cycles a pass (2.4).  One float64 source at 201^3: 15.6 -> 4.3
-// ms with the one-octant update; a float32 one at 65^3: 0.91 -> 0.68 ms.
+// Same passes, same order, same values as k_column.  Bound in float32 by VALU
+// issue where a batch fills the chip (first sweep of 50 sources at 201^3: 490
+// instructions a layer of a patch, its 2.4 passes among them, 79 % of the issue
+// rate), else by the chain of a patch's layers: in float64 15 passes a layer,
+// the 8 + 8 nodes of a patch's longest chain.  A solve on 8 x 8 patches by
+// k_column and so: one float64 source at 201^3 4.0 and 3.35 ms, one float32
+// source at 65^3 0.67 and 0.58, 50 at 201^3 21.4 and 14.3.
 template <typename R, bool FAST, bool SHIFT>
 __global__ void __launch_bounds__(64)
 k_walk8(ColArgs<R> a)
@@ -1334,26 +1335,29 @@ k_walk8(ColArgs<R> a)
     }
 }
 
-// Fixed-point check after sweep a.verify of the column walk.  One thread
-// per free node evaluates the node update on the field as it stands -- the
-// walk's own col_update on the same stencil, in the same arithmetic -- and
-// a node whose value would move marks its patch and its slot.  Nothing is
-// written to the field.  At a fixed point no node moves whatever the order,
-// so a slot with no marked node is where any further sweep would leave it.
+// Fixed-point check after sweep a.verify of the column walk: every free node
+// that could still move has its update evaluated on the field as it stands --
+// the walk's own col_update on the same stencil, in the same arithmetic -- and
+// one whose value would move marks its patch and its slot.  Which nodes could
+// (all, or after a slot's first sweep those with a late input not above them)
+// is found by a look down each column; they are queued per wavefront and
+// evaluated 64 at a time.  Nothing is written to the field.  At a fixed point
+// no node moves whatever the order, so a slot with no marked node is where any
+// further sweep would leave it.
 template <typename R, bool FAST, bool SHIFT>
 __global__ void __launch_bounds__(256) k_verify_mark(ColArgs<R> a)
 {
     const int iter = a.iterp ? __hip_atomic_load(a.iterp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : a.iter;
     if (!a.born && iter != a.verify) return;
-    // one thread per (slot, theta, phi) column walks the layers top down with
-    // the radial window (two above, the node, two below) in registers, so each
-    // value comes from HBM about once, and looks for nodes to evaluate: few
-    // are, scattered over the lanes, so they are queued per wavefront and
-    // evaluated 64 at a time.  The look is bound by latency, so a lane reads
-    // only the inputs that can be late, and B layers' at once (float32, the
-    // first check of 50 fields at 201^3 / 64 at 321^3: 3.1 / 14.4 ms with every
-    // stencil read and evaluated in place, 2.1 / 10.5 with the queue, 1.4 / 6.6
-    // so; a copy of the fields takes 0.7 / 3.6).
+    // a thread looks down the layers of one (slot, theta, phi) column, the
+    // radial window (two above, the node, two below) in registers, so each
+    // value comes from HBM about once.  Few nodes need evaluating, scattered
+    // over the lanes: hence the queue.  The look is bound by latency, so a lane
+    // reads only the inputs that can be late, and B layers' at once (float32,
+    // the first check of 50 fields at 201^3 / 64 at 321^3: 3.1 / 14.4 ms with
+    // every stencil read and evaluated in place, 2.1 / 10.5 with the queue,
+    // 1.4 / 6.6 so; the former 1.2 since doubtful nodes take eight octants at
+    // once; a copy of the fields takes 0.7 / 3.6).
     const size_t NL = (size_t)a.nnx * a.nnz, N = NL * a.nnr, NW = (N + 31) / 32;
     const int np = a.npx * a.npz;
     const R inf = Lim<R>::inf();
@@ -3428,7 +3432,7 @@ static int sweep_kernel(const fmm3d_ctx* c, int k, bool engine)
 // Whether k_walk8 walks the columns: one node per lane, and 32-bit byte
 // offsets within a layer.  Larger layers take k_column's 8 x 8 form, whose
 // addresses are 64-bit ones (a float64 source at 201^3: 4.0 ms against 3.35; 50
-// float32 ones: 22.5 against 15.3).
+// float32 ones: 21.4 against 14.3).
 template <typename R> static bool column_one_node(const fmm3d_ctx* c, const ColArgs<R>& a)
 {
     return c->one_node && a.px == 8 && a.pz == 8 && (size_t)a.nnx * a.nnz * sizeof(R) <= 0xffffffffu;

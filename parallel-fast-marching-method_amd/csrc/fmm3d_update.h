@@ -47,11 +47,11 @@ template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return _
 // is 2^8 of them.  Where an axis' term is not certain, the octant without it
 // is evaluated too, and where both sides of an axis count, the octants of
 // either (float32: all eight in either case), so that every value is the
-// minimum over all eight octants to the last bit.  Measured against eight octants each time: 6 % of the wavefronts'
-// passes need more than one in the first sweep of 50 float32 plane waves at
-// 201^3, which went from 5.55 to 3.53 G VALU instructions; in k_column, eight
-// float64 sources at 31x110x140 went from 9.0 to 5.4 ms and a local source at
-// 61^3 from 53 to 30 ms.
+// minimum over all eight octants to the last bit.  Measured against eight
+// octants each time: 6 % of the wavefronts' passes need more than one in the
+// first sweep of 50 float32 plane waves at 201^3, which went from 5.55 to 3.33
+// G VALU instructions; in k_column, eight float64 sources at 31x110x140 went
+// from 9.0 to 5.4 ms and a local source at 61^3 from 53 to 30 ms.
 
 // The octant of one side per axis (ord 0: none; t1, t2 relative to a common
 // time), its solution and the axes whose term is not certain (bits).
