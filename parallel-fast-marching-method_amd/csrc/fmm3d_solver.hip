@@ -3223,49 +3223,52 @@ __global__ void k_pack_rows(int nr, int64_t rcap, const int32_t* __restrict__ co
 // born: each slot's first sweep, or null (sweep 1).  Slots whose layers are
 // shorter than two cache lines are not placed on one XCD (their fields share
 // lines beyond the first and last layer).
-__global__ void __launch_bounds__(256) k_next_sweep(int* p, int step, int iter, int n, int layer_nodes, const int* __restrict__ on,
-                                                    const int* __restrict__ lastchg, const int* __restrict__ born,
-                                                    int* __restrict__ act)
+__global__ void __launch_bounds__(1024) k_next_sweep(int* p, int step, int iter, int n, int layer_nodes, const int* __restrict__ on,
+                                                     const int* __restrict__ lastchg, const int* __restrict__ born,
+                                                     int* __restrict__ act)
 {
-    __shared__ int part[2][4];
-    const int t = threadIdx.x, w = t >> 6;
+    __shared__ int total[2];        // walked slots: others (0), fresh ones (1)
+    __shared__ int part[2][2][16];  // by parity of the round, per kind: each wavefront's
+    const int t = threadIdx.x, w = t >> 6, nt = blockDim.x;
     const int it = step ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + step : iter;
-    auto walks = [&](int q) { return q < n && on[q] && lastchg[q] >= it - 1; };
-    auto fresh = [&](int q) { return (born ? born[q] : 1) == it; };
-    // per round of 256 slots, the walked fresh ones (kind 1) and others (kind
-    // 0) before thread t's
-    auto count = [&](int q, int kind, int& before, int& all) {
-        const bool a = walks(q) && fresh(q) == (kind != 0);
-        const unsigned long long m = __ballot(a);
-        __syncthreads();
-        if ((t & 63) == 0) part[kind][w] = __popcll(m);
-        __syncthreads();
-        before = __popcll(m & ((1ull << (t & 63)) - 1));
-        for (int j = 0; j < w; ++j) before += part[kind][j];
-        all = part[kind][0] + part[kind][1] + part[kind][2] + part[kind][3];
-        return a;
-    };
-    int nfresh = 0, nold = 0;
-    for (int q0 = 0; q0 < n; q0 += 256) {
-        int before, all;
-        count(q0 + t, 1, before, all);
-        nfresh += all;
-        count(q0 + t, 0, before, all);
-        nold += all;
+    // -1 not walked, else the kind
+    auto kind = [&](int q) { return q < n && on[q] && lastchg[q] >= it - 1 ? ((born ? born[q] : 1) == it ? 1 : 0) : -1; };
+    if (t < 2) total[t] = 0;
+    __syncthreads();   // every thread has read the counter, too
+    int cnt[2] = { 0, 0 };
+    for (int q = t; q < n; q += nt) {
+        const int k = kind(q);
+        cnt[0] += k == 0;
+        cnt[1] += k == 1;
     }
+    if (cnt[0]) atomicAdd(total, cnt[0]);
+    if (cnt[1]) atomicAdd(total + 1, cnt[1]);
+    __syncthreads();
+    const int nfresh = total[1], nold = total[0];
     const int nlocal = layer_nodes >= 64 ? nfresh & ~7 : 0, nspread = nold + nfresh - nlocal;
-    int f = 0, o = 0;
-    for (int q0 = 0; q0 < n; q0 += 256) {
-        int before, all;
-        if (count(q0 + t, 1, before, all)) {
-            const int i = f + before;   // the first nlocal of them are the local ones
-            act[2 + (i < nlocal ? nspread + i : nold + i - nlocal)] = q0 + t;
+    // in slot order, nt at a time: the first nlocal fresh ones are the local ones
+    int done[2] = { 0, 0 };
+    for (int q0 = 0, par = 0; q0 < n; q0 += nt, par ^= 1) {
+        const int k = kind(q0 + t);
+        unsigned long long m[2];
+        for (int j = 0; j < 2; ++j) {
+            m[j] = __ballot(k == j);
+            if ((t & 63) == 0) part[par][j][w] = __popcll(m[j]);
         }
-        f += all;
-        if (count(q0 + t, 0, before, all)) act[2 + o + before] = q0 + t;
-        o += all;
+        __syncthreads();
+        int i = 0;
+        for (int j = 0; j < 2; ++j) {
+            int before = done[j] + __popcll(m[j] & ((1ull << (t & 63)) - 1));
+            for (int v = 0; v < nt >> 6; ++v) {
+                const int c = part[par][j][v];
+                before += v < w ? c : 0;
+                done[j] += c;
+            }
+            if (k == j) i = before;
+        }
+        if (k == 0) act[2 + i] = q0 + t;
+        if (k == 1) act[2 + (i < nlocal ? nspread + i : nold + i - nlocal)] = q0 + t;
     }
-    __syncthreads();   // every thread has read the counter
     if (t == 0) {
         act[0] = nspread;
         act[1] = nlocal;
@@ -3578,6 +3581,14 @@ static hipError_t launch_verify(fmm3d_ctx* c, const ColArgs<R>& a)
     return hipGetLastError();
 }
 
+// k_next_sweep over the slots of a
+template <typename R>
+static void next_sweep(fmm3d_ctx* c, const ColArgs<R>& a, int* p, int step, int iter)
+{
+    k_next_sweep<<<1, a.nslots <= 256 ? 256 : 1024, 0, c->stream>>>(p, step, iter, a.nslots, a.nnx * a.nnz, a.slot_on,
+                                                                     a.lastchg, a.born, c->sl.act);
+}
+
 template <typename R, bool FAST, bool SHIFT>
 static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bool engine = false)
 {
@@ -3601,7 +3612,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
             // before each sweep that lists the slots
             a.act = kd == 1 && a.nslots >= 8 && column_one_node(c, a) ? c->sl.act : nullptr;
             if (a.act)
-                k_next_sweep<<<1, 256, 0, c->stream>>>(nullptr, 0, k + j, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, a.act);
+                next_sweep(c, a, nullptr, 0, k + j);
             if (c->timing) HIPCHK(c, hipEventRecord(c->kev[2 * j], c->stream));
             hipError_t le = launch_column<R, FAST, SHIFT>(c, a, blocks, kd);
             HIPCHK(c, le);
@@ -3654,7 +3665,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
             e = launch_column<R, FAST, SHIFT>(c, a, blocks, kind);
             if (e == hipSuccess && kind == 1 && a.verify > 0 && c->walk_alt != 1) e = launch_verify<R, FAST, SHIFT>(c, a);
             if (e == hipSuccess) {
-                k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 1, 0, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
+                next_sweep(c, a, c->d_iter, 1, 0);
                 e = hipGetLastError();
             }
         }
@@ -3670,7 +3681,7 @@ static int launch_chunk(fmm3d_ctx* c, ColArgs<R> a, int blocks, int n, int k, bo
         }
         c->g_sig = sig;
     }
-    k_next_sweep<<<1, 256, 0, c->stream>>>(c->d_iter, 0, k, a.nslots, a.nnx * a.nnz, a.slot_on, a.lastchg, a.born, c->sl.act);
+    next_sweep(c, a, c->d_iter, 0, k);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
     c->stats.kernel_launches += n;
